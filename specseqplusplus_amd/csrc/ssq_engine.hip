@@ -91,6 +91,7 @@ struct Dev {
   uint8_t* flag;       // scratch per-cell flag (clear / negative)
   uint32_t* piv;       // row -> column
   uint32_t* leftone;   // row -> leftmost column containing it
+  uint32_t* app;       // bit per row: its pivot is the apparent one (set by the init passes)
   int32_t* work[6];    // W0, W1, A0, A1, long list, huge list
   uint32_t* gbits;     // huge-column bit sets: one region of gspan bits per k_add_huge workgroup
   int32_t gspan;       // rows covered by one region
@@ -103,7 +104,7 @@ struct Dev {
   unsigned long long* stats;  // counters at cw::kStats
   uint32_t* err;
   int32_t short_max;    // largest |a|+|b| merged in a wave's LDS (<= kTile)
-  int32_t long_window;  // rows covered by the long-column bit set (<= kLongBits)
+  int32_t long_window;  // rows covered by the long-column bit set (<= kLongBits, a multiple of 128)
 };
 
 // Word offsets in the per-call counter block (64 x uint32 in device memory).
@@ -310,6 +311,22 @@ __global__ void k_dual_init_from_primal(int64_t n, const int64_t* colptr, const 
   }
 }
 
+
+// Bit set of the rows that have a pivot, taken when only the apparent pairs have been entered.
+// A wavefront turns 256 rows into four 64-bit words (the bit set is padded to whole ones).
+__global__ void k_apparent_bits(int64_t n, const uint32_t* piv, uint64_t* app) {
+  const int lane = lane_id();
+  const int64_t waves = (int64_t)gridDim.x * (blockDim.x / kWave);
+  for (int64_t w = (int64_t)blockIdx.x * (blockDim.x / kWave) + threadIdx.x / kWave; w * 256 < n; w += waves) {
+    uint64_t m[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const int64_t r = w * 256 + j * kWave + lane;
+      m[j] = __ballot(r < n && piv[r] != kEmpty);
+    }
+    if (lane < 4) app[w * 4 + lane] = lane == 0 ? m[0] : lane == 1 ? m[1] : lane == 2 ? m[2] : m[3];
+  }
+}
 
 __device__ __forceinline__ int32_t wave_max(int32_t v) {
   for (int d = kWave / 2; d > 0; d >>= 1) v = max(v, __shfl_xor(v, d, kWave));
@@ -727,47 +744,31 @@ __global__ void __launch_bounds__(kWave * kAddWaves) k_add(Dev d, int r, int32_t
 // Long columns of an add round: one workgroup per column.  While the column's rows lie in a
 // window of kLongBits rows below its low, it is kept as a bit set in LDS: adding a pivot
 // toggles the pivot's rows (LDS atomics) and the new low is the highest set bit, found by a
-// block-wide scan downwards from the old low.  This reads only the pivot per addition
-// (a sorted merge reads and writes the whole running column).  A pivot with rows below the
-// window sends the column back to sorted form and tiled merges.
+// block-wide scan downwards from the old low.  This reads only the pivots (a sorted merge reads
+// and writes the whole running column).  A pivot with rows below the window sends the column to
+// k_add_huge.
+//
+// Several pivots per step.  The additions of a chase wait on one another only through the rows
+// they toggle: any pivot of a set row may be added at any time, as every such pivot is a column
+// to the left, and the pairs do not depend on the order or the number of such additions.  A step
+// therefore takes the pivots of all set rows near the low whose pivot is an apparent pair
+// (pick_pivots) and toggles them together.  The low's own pivot is always among them, so the low
+// falls with every step; a row that two of them toggle is set again and met by a later step.
+// Apparent rows are chosen because at most one of them belongs to each leftmost column: the
+// other rows that such a column's block shares with the running column (most additions clear
+// nine and more rows at the top) are cleared by that one addition and must not bring pivots of
+// their own.  A low whose pivot is not apparent is added alone, and the reach starts again: such
+// pivots bring back rows that were cleared ahead of them (alpha complexes: 7 times the additions
+// without that).
+// What it gives: one addition at a time waits for two dependent loads and two barriers (2.1 us);
+// a step takes about 12 us for 22 pivots.  A 1,700-point torus at its 30th distance percentile
+// (longest chase 28,400 additions): k_add_huge 95 -> 46 ms; a 777-point one (1.1 M cells,
+// anti-transposed): k_add_long 3.3 -> 0.8 ms, k_add_huge 6.9 -> 2.5 ms.
 constexpr int kLongBits = 1 << 19;
 constexpr int kLongWords = kLongBits / 32;
 constexpr int kLongThreads = 512;
 constexpr int kHugeGroups = 256;        // k_add_huge workgroups, one device bit set region each
 constexpr int32_t kHugeBits = 1 << 27;  // rows of one region (16 MiB)
-
-__device__ __forceinline__ int32_t block_max_i32(int32_t v, int32_t* scratch) {
-  v = wave_max(v);
-  const int w = threadIdx.x / kWave;
-  __syncthreads();
-  if (lane_id() == 0) scratch[w] = v;
-  __syncthreads();
-  int32_t m = scratch[0];
-  for (int k = 1; k < kLongThreads / kWave; k++) m = max(m, scratch[k]);
-  return m;
-}
-
-// Top two of distinct values (-1 = none): (a1 > a2) merged with (b1 > b2).
-__device__ __forceinline__ void top2_merge(int32_t& a1, int32_t& a2, int32_t b1, int32_t b2) {
-  a2 = max(min(a1, b1), max(a2, b2));
-  a1 = max(a1, b1);
-}
-__device__ __forceinline__ void block_top2(int32_t& v1, int32_t& v2, int32_t* scratch) {
-  for (int k = kWave / 2; k > 0; k >>= 1) {
-    const int32_t o1 = __shfl_xor(v1, k, kWave), o2 = __shfl_xor(v2, k, kWave);
-    top2_merge(v1, v2, o1, o2);
-  }
-  const int w = threadIdx.x / kWave;
-  __syncthreads();
-  if (lane_id() == 0) {
-    scratch[2 * w] = v1;
-    scratch[2 * w + 1] = v2;
-  }
-  __syncthreads();
-  v1 = scratch[0];
-  v2 = scratch[1];
-  for (int k = 1; k < kLongThreads / kWave; k++) top2_merge(v1, v2, scratch[2 * k], scratch[2 * k + 1]);
-}
 
 __device__ __forceinline__ int32_t block_excl_scan(int32_t v, int32_t* scratch, int32_t* total) {
   const int w = threadIdx.x / kWave;
@@ -784,17 +785,142 @@ __device__ __forceinline__ int32_t block_excl_scan(int32_t v, int32_t* scratch, 
   return base + incl - v;
 }
 
+// The pivots of one step (LDS).  Three slots in turn: a slot is cleared while the one before it
+// is being filled, two barriers after its last read.
+constexpr int kPicks = 512;                        // pivots of one step
+constexpr int kPickWords = 4 * kLongThreads;       // LDS words that a step looks at: one uint4 per thread
+constexpr int32_t kReachMin = 31;                  // rows below the low that the first step picks from
+struct __align__(16) Pick {
+  int64_t off;
+  int32_t len;
+};
+struct Picks {
+  Pick list[kPicks];
+  uint32_t count[3];
+  uint32_t top[3];  // 0: no set row seen, else ((row - row0) + 1) << 1 | its pivot is in the list
+  int32_t minw;     // lowest region word that a pivot in the list reached (k_add_huge)
+};
+
+// The apparent-pivot bits of the LDS words that this thread looks at from word base down.
+__device__ __forceinline__ uint4 pick_mask(const Dev& d, int32_t base, int32_t row0) {
+  const int32_t g = (base >> 2) - (int32_t)threadIdx.x;
+  const int32_t r0 = row0 + 128 * g;  // rows below 0 are never set
+  return g >= 0 && r0 >= 0 ? *(const uint4*)(d.app + (r0 >> 5)) : make_uint4(0u, 0u, 0u, 0u);
+}
+
+// One look at the window: LDS words [base - kPickWords, base] (base >= the highest nonzero word),
+// thread t at words 4 * ((base >> 2) - t) .. + 3.  row0 (a multiple of 128) is the row of word 0.
+// Pivots of apparent set rows >= from go to the list, the highest set row to top[slot].  Pivots
+// with rows below `lo` are left out.  No pivot needs comparing with the running column c: an
+// apparent pivot is the leftmost column with its row, and c is a sum of columns up to c, so it
+// lies left of c.
+__device__ __forceinline__ void pick_pivots(const Dev& d, const uint32_t* bits, int32_t base, int32_t row0,
+                                            int32_t from, int32_t lo, const uint4& a, Picks* P, int slot,
+                                            uint32_t* max_len) {
+  if (threadIdx.x == 0) {
+    const int next = slot == 2 ? 0 : slot + 1;
+    P->count[next] = 0;
+    P->top[next] = 0;
+  }
+  const int32_t g = (base >> 2) - (int32_t)threadIdx.x;
+  uint4 v = make_uint4(0u, 0u, 0u, 0u);
+  if (g >= 0) v = ((const uint4*)bits)[g];
+  const bool any = (v.x | v.y | v.z | v.w) != 0u;
+  const uint64_t who = __ballot(any);
+  if (!who) return;
+  uint32_t enc = 0;
+  if (any) {
+    const int32_t r0 = row0 + 128 * g;  // a multiple of 128; a set row is >= 0, so r0 is
+    const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+    int32_t top = 0;
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      if (w[j]) top = 32 * j + 31 - __clz(w[j]);
+    enc = (uint32_t)(128 * g + top + 1) << 1;
+    if (r0 + top >= from) {
+      const uint32_t cand[4] = {v.x & a.x, v.y & a.y, v.z & a.z, v.w & a.w};
+#pragma unroll
+      for (int j = 3; j >= 0; j--) {
+        uint32_t m = cand[j];
+        while (m) {
+          const int h = 31 - __clz(m);
+          m &= ~(1u << h);
+          const int32_t row = r0 + 32 * j + h;
+          if (row < from) break;
+          const PivMeta pm = d.pivmeta[row];
+          if (pm.first < lo) continue;
+          const uint32_t at = atomicAdd(&P->count[slot], 1u);
+          if (at < (uint32_t)kPicks) {
+            P->list[at].off = pm.off;
+            P->list[at].len = pm.len;
+            atomicMin(&P->minw, (pm.first - lo) >> 5);
+            *max_len = max(*max_len, (uint32_t)pm.len);
+            if (32 * j + h == top) enc |= 1u;
+          }
+        }
+      }
+    }
+  }
+  // rows descend with the thread: the first lane with a set row holds the wavefront's highest
+  const uint32_t best = (uint32_t)__builtin_amdgcn_readlane((int)enc, __ffsll((unsigned long long)who) - 1);
+  if (lane_id() == 0) atomicMax(&P->top[slot], best);
+}
+
+// How far below the low the next step picks: twice as far, unless the n pivots of this one
+// outnumber all additions before it (a chase that ends early should not have added many pivots
+// below its last low).
+__device__ __forceinline__ int32_t next_reach(int32_t reach, uint32_t n, uint32_t chain) {
+  return n <= max(chain, 1u) ? min(2 * reach, kLongBits) : max(reach / 2, kReachMin);
+}
+
+// The highest set row at or below word base, with the pivots near it, looking further down until
+// one is found or the window ends.  mask: pick_mask of base, loaded ahead (the next base is known
+// before the rows of a step are toggled).  Returns top[] (uniform); *slot moves on.
+__device__ __forceinline__ uint32_t next_step(const Dev& d, const uint32_t* bits, int32_t base, int32_t row0,
+                                              int32_t reach, int32_t lo, int32_t minrow, uint4 mask, Picks* P,
+                                              int* slot, uint32_t* count, uint32_t* max_len) {
+  for (;;) {
+    const int s = *slot;
+    const int32_t from = max(minrow, row0 + 32 * base + 31 - reach);
+    pick_pivots(d, bits, base, row0, from, lo, mask, P, s, max_len);
+    __syncthreads();
+    *slot = s == 2 ? 0 : s + 1;
+    const uint32_t t = (uint32_t)__builtin_amdgcn_readfirstlane((int)P->top[s]);
+    *count = (uint32_t)__builtin_amdgcn_readfirstlane((int)P->count[s]);
+    base = (base & ~3) - kPickWords + 3;
+    if (t || base < 0) return t;
+    mask = pick_mask(d, base, row0);
+  }
+}
+
+// f(row - lo) for every row of a pivot, spread over kThreads threads with kU loads in flight each.
+template <int kThreads, int kU, typename F>
+__device__ __forceinline__ void toggle_rows(const int32_t* B, int32_t len, int t, int32_t lo, F f) {
+  for (int32_t k0 = t; k0 < len; k0 += kThreads * kU) {
+    int32_t x[kU];
+#pragma unroll
+    for (int u = 0; u < kU; u++) {
+      const int32_t k = k0 + u * kThreads;
+      x[u] = k < len ? B[k] - lo : -1;
+    }
+#pragma unroll
+    for (int u = 0; u < kU; u++)
+      if (x[u] >= 0) f(x[u]);
+  }
+}
+
 __global__ void __launch_bounds__(kLongThreads) k_add_long(Dev d, int r, int32_t minrow) {
-  __shared__ uint32_t bits[kLongWords];
-  __shared__ int32_t red[2 * (kLongThreads / kWave)];
-  __shared__ int32_t sh_count, sh_flag;
+  __shared__ __align__(16) uint32_t bits[kLongWords];
+  __shared__ Picks picks;
+  __shared__ int32_t red[kLongThreads / kWave];
+  __shared__ int32_t sh_flag;
   __shared__ int64_t sh_off;
   __shared__ int32_t sh_cap;
   const int nx = (r + 1) & 1;
   const int tid = threadIdx.x;
   const uint32_t cnt = d.ctr[cw::kLong];
   const int32_t* list = d.work[4];
-  unsigned long long n_add = 0, n_dense = 0, n_dbytes = 0, n_tiled = 0;
+  unsigned long long n_add = 0, n_bytes = 0;
   uint32_t max_chain = 0, max_len = 0;
 
   for (int64_t it = blockIdx.x; it < cnt; it += gridDim.x) {
@@ -803,179 +929,66 @@ __global__ void __launch_bounds__(kLongThreads) k_add_long(Dev d, int r, int32_t
     int32_t a_cap = d.cap[c];
     int32_t a_len = d.len[c];
     int32_t l = d.low[c];
-    bool to_huge = false;
-    const int32_t lo = l - d.long_window + 1;  // window [lo, l] of the bit set
-    bool dense = d.pool[a_off] >= lo;
-    bool failed = false;
-    uint32_t chain = 0;
-    // a2: the running column's largest row below l (-1 none, kUnknown not known).  When it
-    // differs from the pivot's, the larger of the two is the next low, so that low's pivot
-    // is fetched while the current addition is still toggling rows.
-    constexpr int32_t kUnknown = -3;
-    int32_t a2 = a_len >= 2 ? d.pool[a_off + a_len - 2] : -1;
-    int32_t spec_row = -2;
-    uint32_t spec_p = kEmpty;
-    PivMeta spec_pm{};
-    if (dense) {
-      const int32_t nw = ((l - lo) >> 5) + 1;
-      for (int32_t w = tid; w < nw; w += kLongThreads) bits[w] = 0u;
+    bool to_huge = false, failed = false;
+    const int32_t lo = (l & ~127) + 128 - d.long_window;  // the bit set holds rows [lo, l]
+    if (d.pool[a_off] < lo) {
+      // the column's rows leave the window: k_add_huge takes it if it has a pivot to add
+      const uint32_t p = d.piv[l];
+      to_huge = p != kEmpty && p < (uint32_t)c;
+    } else {
+      uint4* b4 = (uint4*)bits;
+      for (int32_t k = tid; k < d.long_window / 128; k += kLongThreads) b4[k] = make_uint4(0u, 0u, 0u, 0u);
+      if (tid < 3) picks.count[tid] = picks.top[tid] = 0;
       __syncthreads();
       const int32_t* A = d.pool + a_off;
       for (int32_t k = tid; k < a_len; k += kLongThreads) {
         const int32_t x = A[k] - lo;
         atomicOr(&bits[x >> 5], 1u << (x & 31));
       }
-      if (tid == 0) sh_count = a_len;
       __syncthreads();
-    }
-    for (;;) {
-      // the chase state is uniform across the workgroup: scalar loads
-      l = __builtin_amdgcn_readfirstlane(l);
-      uint32_t p;
-      PivMeta pm;
-      if (l == spec_row) {
-        p = spec_p;
-        pm = spec_pm;
-      } else {
-        p = d.piv[l];
-        pm = d.pivmeta[l];
+      uint32_t chain = 0;
+      int32_t reach = kReachMin;
+      int slot = 0;
+      uint4 mask = pick_mask(d, (l - lo) >> 5, lo);
+      for (;;) {
+        uint32_t n;
+        const uint32_t t = next_step(d, bits, (l - lo) >> 5, lo, reach, lo, minrow, mask, &picks, &slot, &n, &max_len);
+        l = t ? lo + (int32_t)(t >> 1) - 1 : -1;
+        if (l < 0 || l < minrow) break;  // every row cancelled, or the low is below the page
+        mask = pick_mask(d, (l - lo) >> 5, lo);
+        if (t & 1u) {
+          n = min(n, (uint32_t)kPicks);
+          reach = next_reach(reach, n, chain);
+          for (uint32_t e = tid / kWave; e < n; e += kLongThreads / kWave) {
+            const int32_t len = picks.list[e].len;
+            toggle_rows<kWave, 8>(d.pool + picks.list[e].off, len, lane_id(), lo, [&](int32_t x) {
+              atomicXor(&bits[x >> 5], 1u << (x & 31));
+            });
+            n_bytes += 4ull * (unsigned long long)len + 24ull;  // the pivot read; the bit set is in LDS
+          }
+          chain += n;
+        } else {
+          const uint32_t p = (uint32_t)__builtin_amdgcn_readfirstlane((int)d.piv[l]);
+          if (p == kEmpty || p >= (uint32_t)c) break;
+          const PivMeta pm = d.pivmeta[l];
+          const bool app = (d.app[l >> 5] >> (l & 31)) & 1u;
+          if (pm.first < lo) {  // the pivot reaches below the window
+            to_huge = true;
+            break;
+          }
+          toggle_rows<kLongThreads, 16>(d.pool + pm.off, pm.len, tid, lo, [&](int32_t x) {
+            atomicXor(&bits[x >> 5], 1u << (x & 31));
+          });
+          if (tid < kWave) n_bytes += 4ull * (unsigned long long)pm.len + 24ull;
+          max_len = max(max_len, (uint32_t)pm.len);
+          reach = app ? next_reach(reach, 1u, chain) : kReachMin;
+          chain += 1;
+        }
+        __syncthreads();
       }
-      p = (uint32_t)__builtin_amdgcn_readfirstlane((int)p);
-      if (p == kEmpty || p >= (uint32_t)c) break;
-      const int32_t b_len = __builtin_amdgcn_readfirstlane(pm.len);
-      const int32_t b_first = __builtin_amdgcn_readfirstlane(pm.first);
-      const int32_t b2 = __builtin_amdgcn_readfirstlane(pm.second);
-      const int64_t b_off = (int64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(pm.off & 0xffffffff)) |
-                            ((int64_t)__builtin_amdgcn_readfirstlane((int)(pm.off >> 32)) << 32);
-      const int32_t* B = d.pool + b_off;
-      if (dense && b_first < lo) {
-        // leave the bit set: write the column back in sorted form
-        int32_t W = ((l - lo) >> 5) + 1, total;
-        const int32_t per = (W + kLongThreads - 1) / kLongThreads;
-        const int32_t w0 = min(W, tid * per), w1 = min(W, w0 + per);
-        int32_t pc = 0;
-        for (int32_t w = w0; w < w1; w++) pc += __popc(bits[w]);
-        const int32_t pos0 = block_excl_scan(pc, red, &total);
-        if (tid == 0) {
-          int64_t o = a_off;
-          int32_t cp = a_cap;
-          sh_flag = 1;
-          if (total > cp && !store_alloc(d, total, &o, &cp)) sh_flag = 0;
-          sh_off = o;
-          sh_cap = cp;
-        }
-        __syncthreads();
-        if (!sh_flag) { failed = true; break; }
-        a_off = sh_off;
-        a_cap = sh_cap;
-        int32_t* O = d.pool + a_off;
-        int32_t pos = pos0;
-        for (int32_t w = w0; w < w1; w++) {
-          uint32_t x = bits[w];
-          while (x) {
-            const int b = __ffs(x) - 1;
-            O[pos++] = lo + (w << 5) + b;
-            x &= x - 1;
-          }
-        }
-        __threadfence();
-        __syncthreads();
-        a_len = total;
-        dense = false;
-      }
-      int32_t r_len;
-      if (dense) {
-        spec_row = -2;
-        if (a2 != kUnknown && a2 != b2) {
-          const int32_t cand = max(a2, b2);
-          if (cand >= 0 && cand >= minrow) {
-            spec_row = cand;
-            spec_p = d.piv[cand];
-            spec_pm = d.pivmeta[cand];
-          }
-        }
-        // toggle the pivot's rows
-        int32_t delta = 0;
-        constexpr int kU = 16;  // independent loads in flight per thread
-        for (int32_t k0 = tid; k0 < b_len; k0 += kLongThreads * kU) {
-          int32_t x[kU];
-#pragma unroll
-          for (int u = 0; u < kU; u++) {
-            const int32_t k = k0 + u * kLongThreads;
-            x[u] = k < b_len ? B[k] - lo : -1;
-          }
-#pragma unroll
-          for (int u = 0; u < kU; u++)
-            if (x[u] >= 0) {
-              const uint32_t m = 1u << (x[u] & 31);
-              const uint32_t old = atomicXor(&bits[x[u] >> 5], m);
-              delta += (old & m) ? -1 : 1;
-            }
-        }
-        {  // the wavefront's sum of the changes by bit planes: |delta| <= 1024 (a pivot in the
-           // bit set has at most kLongBits rows over kLongThreads threads), offset to >= 0
-          const uint32_t u = (uint32_t)(delta + 2048);
-          uint32_t sum = 0;
-#pragma unroll
-          for (int b = 0; b < 12; b++) sum += (uint32_t)__popcll(__ballot((u >> b) & 1u)) << b;
-          if (lane_id() == 0) atomicAdd(&sh_count, (int32_t)sum - 2048 * kWave);
-        }
-        __syncthreads();
-        r_len = sh_count;
-        // new low and the row below it: the two highest set bits, scanning down from the old
-        // low's word.  Wavefront 0 alone scans, 64 words per step (one ballot finds the
-        // nonzero words), and publishes them; the second is looked for up to 8 steps past the
-        // first.  Two barriers per addition:
-        // every read of this step's LDS values happens before the second, every write of the
-        // next step after it.
-        if (tid < kWave) {
-          const int lane = tid;
-          int32_t t1 = -1, t2 = -1, past = 0;
-          int32_t base = r_len > 0 ? (l - lo) >> 5 : -1;  // r_len is uniform (read from LDS)
-          for (; base >= 0; base -= kWave) {  // t1, t2 are uniform in the wavefront: so are the exits
-            // lane k holds word base - k, so rows descend with the lane: the highest rows are
-            // in the first lanes whose words are nonzero, read one word at a time (scalar)
-            const int32_t w = base - lane;
-            const uint32_t m = w >= 0 ? bits[w] : 0u;
-            uint64_t nz = __ballot(m != 0);
-            while (nz && t2 < 0) {
-              const int fl = __ffsll((unsigned long long)nz) - 1;
-              nz &= nz - 1;
-              uint32_t mm = (uint32_t)__builtin_amdgcn_readlane((int)m, fl);
-              const int32_t row0 = lo + ((base - fl) << 5);
-              while (mm && t2 < 0) {
-                const int h = 31 - __clz(mm);
-                mm &= ~(1u << h);
-                if (t1 < 0) t1 = row0 + h;
-                else t2 = row0 + h;
-              }
-            }
-            if (t2 >= 0 || (t1 >= 0 && r_len == 1)) break;
-            if (t1 >= 0 && ++past >= 8) break;
-          }
-          if (lane == 0) {
-            red[0] = t1;
-            red[1] = t2 >= 0 ? t2 : ((base < 0 || r_len <= 1) ? -1 : kUnknown);
-          }
-        }
-        __syncthreads();
-        const int32_t newl = red[0];
-        a2 = red[1];
-        n_dense += 1;
-        n_dbytes += 4ull * (unsigned long long)b_len + 24ull;  // the pivot read; the bit set is in LDS
-        max_len = max(max_len, (uint32_t)(a_len + b_len));
-        chain += 1;
-        a_len = r_len;
-        l = r_len ? newl : -1;
-      } else {
-        // the column's rows leave the window: k_add_huge continues the chase in this round
-        to_huge = true;
-        break;
-      }
-      if (l < 0 || l < minrow) break;
-    }
-    max_chain = max(max_chain, chain);
-    if (!failed && dense) {  // write the bit set back in sorted form
+      n_add += chain;
+      max_chain = max(max_chain, chain);
+      // the bit set back in sorted form
       const int32_t W = l >= 0 ? ((l - lo) >> 5) + 1 : 0;
       int32_t total;
       const int32_t per = (W + kLongThreads - 1) / kLongThreads;
@@ -1034,13 +1047,15 @@ __global__ void __launch_bounds__(kLongThreads) k_add_long(Dev d, int r, int32_t
     }
     __syncthreads();
   }
-  if (tid == 0 && (n_add || n_dense)) {
-    atomicAdd(&d.stats[0], n_add + n_dense);
-    atomicAdd(&d.stats[2], n_tiled);
-    atomicAdd(&d.stats[3], n_dense);
-    atomicAdd(&d.stats[4], n_dbytes);
-    atomicMax(&d.ctr[cw::kChain], max_chain);
+  max_len = (uint32_t)wave_max((int32_t)max_len);
+  if (lane_id() == 0 && n_bytes) {  // every wavefront's own pivots
+    atomicAdd(&d.stats[4], n_bytes);
     atomicMax(&d.ctr[cw::kChain + 1], max_len);
+  }
+  if (tid == 0 && n_add) {
+    atomicAdd(&d.stats[0], n_add);
+    atomicAdd(&d.stats[3], n_add);
+    atomicMax(&d.ctr[cw::kChain], max_chain);
   }
 }
 
@@ -1053,9 +1068,9 @@ __global__ void __launch_bounds__(kLongThreads) k_add_long(Dev d, int r, int32_t
 // below it that nothing waits for.  The new low is looked for in the window.  Only when the
 // window has emptied does the workgroup wait for its global toggles, find the tail's highest
 // row through the summary, and move the window down onto it (reading those words into LDS and
-// clearing them).  The next pivot is fetched while the current one is toggled, whenever the
-// column's second row is known (the next low is then the larger of the two second rows when
-// they differ).  A region is all zero between columns.  A pivot with rows below the region
+// clearing them).  What bounds it: the toggles below the window, one device atomic per row, each
+// lane another line: 1.75 ns per row and workgroup (0.2-0.3 ns in the window).
+// A region is all zero between columns.  A pivot with rows below the region
 // sends the column to sorted form and tiled merges, ping-ponging between the column's own slot
 // and one scratch slot.
 __device__ __forceinline__ uint32_t gload(const uint32_t* p) {
@@ -1075,38 +1090,6 @@ __device__ __forceinline__ void mark_chunk(uint32_t* summ, int32_t g) {
 }
 __device__ __forceinline__ bool chunk_marked(const uint32_t* summ, int32_t ch) {
   return (summ[ch >> 5] >> (ch & 31)) & 1u;
-}
-
-// Wavefront 0: the two highest set bits of the window at or below LDS word top_w (rows
-// wrow0 + 32 * word + bit).  t2 is kUnknown when the window's bottom was reached with t1 only
-// (the tail may hold it) or when it lies more than 8 steps of 64 words below t1.
-constexpr int32_t kUnknown = -3;
-__device__ __forceinline__ void window_top2(const uint32_t* bits, int32_t top_w, int32_t wrow0, int32_t* t1o,
-                                            int32_t* t2o) {
-  const int lane = lane_id();
-  int32_t t1 = -1, t2 = -1, past = 0;
-  int32_t base = top_w;
-  for (; base >= 0; base -= kWave) {  // t1, t2 are uniform in the wavefront: so are the exits
-    const int32_t w = base - lane;    // lane k holds word base - k: rows descend with the lane
-    const uint32_t m = w >= 0 ? bits[w] : 0u;
-    uint64_t nz = __ballot(m != 0);
-    while (nz && t2 < 0) {
-      const int fl = __ffsll((unsigned long long)nz) - 1;
-      nz &= nz - 1;
-      uint32_t mm = (uint32_t)__builtin_amdgcn_readlane((int)m, fl);
-      const int32_t row0 = wrow0 + ((base - fl) << 5);
-      while (mm && t2 < 0) {
-        const int h = 31 - __clz(mm);
-        mm &= ~(1u << h);
-        if (t1 < 0) t1 = row0 + h;
-        else t2 = row0 + h;
-      }
-    }
-    if (t2 >= 0) break;
-    if (t1 >= 0 && ++past >= 8) break;
-  }
-  *t1o = t1;
-  *t2o = t2 >= 0 ? t2 : (t1 >= 0 ? kUnknown : -1);
 }
 
 // Wavefront 0: the tail's highest set row below region chunk ch_top + 1 (all global toggles
@@ -1227,11 +1210,12 @@ __device__ __forceinline__ int32_t window_base(int32_t lw) {
 }
 
 __global__ void __launch_bounds__(kLongThreads) k_add_huge(Dev d, int r, int32_t minrow) {
-  __shared__ uint32_t bits[kLongWords];
+  __shared__ __align__(16) uint32_t bits[kLongWords];
   __shared__ uint32_t summ[kSumWords];
   __shared__ int32_t stage[3][kTileBuf];
-  __shared__ int32_t red[2 * (kLongThreads / kWave)];
-  __shared__ int32_t sh_flag, sh_minw, sh_cap;
+  __shared__ Picks picks;
+  __shared__ int32_t red[kLongThreads / kWave];
+  __shared__ int32_t sh_flag, sh_cap;
   __shared__ int64_t sh_off;
   __shared__ uint32_t sh_item;
   const int nx = (r + 1) & 1;
@@ -1253,20 +1237,22 @@ __global__ void __launch_bounds__(kLongThreads) k_add_huge(Dev d, int r, int32_t
     int32_t a_cap = d.cap[c];
     int32_t a_len = d.len[c];
     int32_t l = d.low[c];
-    const int32_t lo = l - d.gspan + 1;  // the region holds rows [lo, l]
+    const int32_t lo = (l & ~127) + 128 - d.gspan;  // the region holds rows [lo, l]
     bool dense = a_len > 0 && d.pool[a_off] >= lo;
     bool failed = false;
     uint32_t chain = 0;
     int64_t t_off = 0;  // scratch slot of the tiled merges (thread 0's copy is used)
     int32_t t_cap = 0;
     int32_t ww0 = window_base((l - lo) >> 5);  // region word of LDS word 0
-    int32_t a2 = kUnknown;                     // the running column's second row
-    int32_t spec_row = -2;
-    uint32_t spec_p = kEmpty;
-    PivMeta spec_pm{};
+    int32_t base = ((l - lo) >> 5) - ww0;      // highest LDS word that may be nonzero
+    int32_t reach = kReachMin;
+    int slot = 0;
+    uint4 mask = dense ? pick_mask(d, base, lo + (ww0 << 5)) : make_uint4(0u, 0u, 0u, 0u);
     if (dense) {
-      for (int32_t k = tid; k < kLongWords; k += kLongThreads) bits[k] = 0u;
+      uint4* b4 = (uint4*)bits;
+      for (int32_t k = tid; k < kLongWords / 4; k += kLongThreads) b4[k] = make_uint4(0u, 0u, 0u, 0u);
       for (int32_t k = tid; k < nsum; k += kLongThreads) summ[k] = 0u;
+      if (tid < 3) picks.count[tid] = picks.top[tid] = 0;
       __syncthreads();
       const int32_t* A = d.pool + a_off;
       for (int32_t k = tid; k < a_len; k += kLongThreads) {
@@ -1278,32 +1264,96 @@ __global__ void __launch_bounds__(kLongThreads) k_add_huge(Dev d, int r, int32_t
           mark_chunk(summ, g);
         }
       }
-      if (tid == 0) sh_minw = (A[0] - lo) >> 5;
+      if (tid == 0) picks.minw = (A[0] - lo) >> 5;
       __threadfence();
       __syncthreads();
-      a2 = a_len >= 2 ? A[a_len - 2] : -1;
     }
-    for (;;) {
-      l = __builtin_amdgcn_readfirstlane(l);
-      uint32_t p;
-      PivMeta pm;
-      if (l == spec_row) {
-        p = spec_p;
-        pm = spec_pm;
+    const auto toggle = [&](int32_t x) {
+      const int32_t g = x >> 5;
+      const uint32_t m = 1u << (x & 31);
+      if (g >= ww0) {
+        atomicXor(&bits[g - ww0], m);
       } else {
-        p = d.piv[l];
-        pm = d.pivmeta[l];  // fetched with the pivot (meaningful only if it exists)
+        gxor(gb + g, m);
+        mark_chunk(summ, g);
       }
-      p = (uint32_t)__builtin_amdgcn_readfirstlane((int)p);
+    };
+    for (;;) {
+      if (dense) {
+        uint32_t n;
+        const int32_t row0 = lo + (ww0 << 5);
+        const uint32_t t = next_step(d, bits, base, row0, reach, lo, minrow, mask, &picks, &slot, &n, &max_len);
+        if (!t) {
+          // the window is empty: wait for the global toggles, take the tail's highest row and
+          // move the window onto it
+          l = -1;
+          if (ww0 == 0) break;
+          __threadfence();
+          __syncthreads();
+          if (tid < kWave) {
+            const int32_t top = tail_top(summ, gb, (ww0 >> 5) - 1, nwords, lo);
+            if (tid == 0) red[0] = top;
+          }
+          __syncthreads();
+          l = red[0];
+          if (l < 0) break;
+          const int32_t lw = (l - lo) >> 5;
+          const int32_t nb = window_base(lw);  // chunk-aligned, below the old window
+          // pull the marked chunks [nb >> 5, lw >> 5] into the (all zero) window
+          const int32_t c0 = nb >> 5, C = (lw >> 5) - c0 + 1;
+          for (int32_t ci = tid; ci < C; ci += kLongThreads) {
+            const int32_t ch = c0 + ci;
+            if (!chunk_marked(summ, ch)) continue;
+            const int32_t ke = min(kChunkWords, nwords - (ch << 5));
+            for (int32_t k = 0; k < ke; k++) {
+              const int32_t g = (ch << 5) + k;
+              const uint32_t x = gload(gb + g);
+              bits[g - nb] = x;
+              if (x) gb[g] = 0u;
+            }
+          }
+          __syncthreads();
+          for (int32_t ci = tid; ci < C; ci += kLongThreads) {  // every pulled chunk is now zero
+            const int32_t ch = c0 + ci;
+            if (chunk_marked(summ, ch)) atomicAnd(&summ[ch >> 5], ~(1u << (ch & 31)));
+          }
+          ww0 = nb;
+          base = lw - nb;
+          mask = pick_mask(d, base, lo + (ww0 << 5));
+          __syncthreads();
+          continue;
+        }
+        l = row0 + (int32_t)(t >> 1) - 1;
+        if (l < minrow) break;
+        base = ((l - lo) >> 5) - ww0;
+        mask = pick_mask(d, base, row0);
+        if (t & 1u) {  // the low's pivot and those of the rows near it
+          n = min(n, (uint32_t)kPicks);
+          reach = next_reach(reach, n, chain);
+          for (uint32_t e = tid / kWave; e < n; e += kLongThreads / kWave) {
+            const int32_t len = picks.list[e].len;
+            toggle_rows<kWave, 8>(d.pool + picks.list[e].off, len, lane_id(), lo, toggle);
+            n_bytes += 4ull * (unsigned long long)len + 24ull;  // the pivot read; the bit set stays on chip
+          }
+          chain += n;
+          n_add += n;
+          __syncthreads();
+          continue;
+        }
+      }
+      // the low's own pivot alone
+      l = __builtin_amdgcn_readfirstlane(l);
+      const uint32_t p = (uint32_t)__builtin_amdgcn_readfirstlane((int)d.piv[l]);
       if (p == kEmpty || p >= (uint32_t)c) break;
+      const PivMeta pm = d.pivmeta[l];
+      const bool app = (d.app[l >> 5] >> (l & 31)) & 1u;
       const int32_t b_len = __builtin_amdgcn_readfirstlane(pm.len);
       const int32_t b_first = __builtin_amdgcn_readfirstlane(pm.first);
-      const int32_t b2 = __builtin_amdgcn_readfirstlane(pm.second);
       const int64_t b_off = (int64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(pm.off & 0xffffffff)) |
                             ((int64_t)__builtin_amdgcn_readfirstlane((int)(pm.off >> 32)) << 32);
       const int32_t* B = d.pool + b_off;
       if (dense && b_first < lo) {  // leave the region: sorted form, then tiled merges
-        if (!huge_write_back(d, gb, summ, bits, lo, ww0, sh_minw, ((l - lo) >> 5) - ww0, &a_off, &a_cap, &a_len,
+        if (!huge_write_back(d, gb, summ, bits, lo, ww0, picks.minw, ((l - lo) >> 5) - ww0, &a_off, &a_cap, &a_len,
                              red, &sh_flag, &sh_off, &sh_cap)) {
           failed = true;
           break;
@@ -1311,106 +1361,14 @@ __global__ void __launch_bounds__(kLongThreads) k_add_huge(Dev d, int r, int32_t
         dense = false;
       }
       if (dense) {
-        spec_row = -2;
-        if (a2 != kUnknown && a2 != b2) {
-          const int32_t cand = max(a2, b2);
-          if (cand >= 0 && cand >= minrow) {
-            spec_row = cand;
-            spec_p = d.piv[cand];
-            spec_pm = d.pivmeta[cand];
-          }
-        }
-        // toggle the pivot's rows
-        constexpr int kU = 16;  // independent loads in flight per thread
-        for (int32_t k0 = tid; k0 < b_len; k0 += kLongThreads * kU) {
-          int32_t x[kU];
-#pragma unroll
-          for (int u = 0; u < kU; u++) {
-            const int32_t k = k0 + u * kLongThreads;
-            x[u] = k < b_len ? B[k] - lo : -1;
-          }
-#pragma unroll
-          for (int u = 0; u < kU; u++)
-            if (x[u] >= 0) {
-              const int32_t g = x[u] >> 5;
-              const uint32_t m = 1u << (x[u] & 31);
-              if (g >= ww0) {
-                atomicXor(&bits[g - ww0], m);
-              } else {
-                gxor(gb + g, m);
-                mark_chunk(summ, g);
-              }
-            }
-        }
-        if (tid == 0) atomicMin(&sh_minw, (b_first - lo) >> 5);
-        __syncthreads();
-        // new low and the row below it, in the window; consecutive additions use alternate
-        // slots of red[], so an addition's slot is rewritten only two barriers after every
-        // thread has read it
-        const int rb = (int)(chain & 1u) * 2;
-        if (tid < kWave) {
-          int32_t t1, t2;
-          window_top2(bits, ((l - lo) >> 5) - ww0, lo + (ww0 << 5), &t1, &t2);
-          if (tid == 0) {
-            red[rb] = t1;
-            red[rb + 1] = t2;
-          }
-        }
-        __syncthreads();
-        int32_t newl = red[rb];
-        a2 = red[rb + 1];
-        if (newl < 0 && ww0 > 0) {
-          // the window is empty: wait for the global toggles, take the tail's highest row and
-          // move the window onto it
-          __threadfence();
-          __syncthreads();
-          if (tid < kWave) {
-            const int32_t t = tail_top(summ, gb, (ww0 >> 5) - 1, nwords, lo);
-            if (tid == 0) red[0] = t;
-          }
-          __syncthreads();
-          newl = red[0];
-          if (newl >= 0) {
-            const int32_t lw = (newl - lo) >> 5;
-            const int32_t nb = window_base(lw);  // chunk-aligned, below the old window
-            // pull the marked chunks [nb >> 5, lw >> 5] into the (all zero) window
-            const int32_t c0 = nb >> 5, C = (lw >> 5) - c0 + 1;
-            for (int32_t ci = tid; ci < C; ci += kLongThreads) {
-              const int32_t ch = c0 + ci;
-              if (!chunk_marked(summ, ch)) continue;
-              const int32_t ke = min(kChunkWords, nwords - (ch << 5));
-              for (int32_t k = 0; k < ke; k++) {
-                const int32_t g = (ch << 5) + k;
-                const uint32_t x = gload(gb + g);
-                bits[g - nb] = x;
-                if (x) gb[g] = 0u;
-              }
-            }
-            __syncthreads();
-            for (int32_t ci = tid; ci < C; ci += kLongThreads) {  // every pulled chunk is now zero
-              const int32_t ch = c0 + ci;
-              if (chunk_marked(summ, ch)) atomicAnd(&summ[ch >> 5], ~(1u << (ch & 31)));
-            }
-            ww0 = nb;
-            __syncthreads();
-            if (tid < kWave) {
-              int32_t t1, t2;
-              window_top2(bits, lw - ww0, lo + (ww0 << 5), &t1, &t2);
-              if (tid == 0) {
-                red[0] = t1;
-                red[1] = t2;
-              }
-            }
-            __syncthreads();
-            newl = red[0];
-            a2 = red[1];
-          }
-        }
+        toggle_rows<kLongThreads, 16>(B, b_len, tid, lo, toggle);
+        if (tid == 0) atomicMin(&picks.minw, (b_first - lo) >> 5);
         n_add += 1;
-        n_bytes += 4ull * (unsigned long long)b_len + 24ull;  // the pivot read; the bit set stays on chip
+        if (tid < kWave) n_bytes += 4ull * (unsigned long long)b_len + 24ull;
         max_len = max(max_len, (uint32_t)b_len);
+        reach = app ? next_reach(reach, 1u, chain) : kReachMin;
         chain += 1;
-        l = newl;
+        __syncthreads();
       } else {
         // tiled merge by wave 0 into the other of two slots: the column's own and one scratch
         // slot, swapped after each addition; the scratch slot is replaced (twice the need)
@@ -1446,7 +1404,7 @@ __global__ void __launch_bounds__(kLongThreads) k_add_huge(Dev d, int r, int32_t
         r_len = red[0];
         n_tiled += 1;
         n_add += 1;
-        n_bytes += 4ull * (unsigned long long)(a_len + b_len + r_len) + 24ull;
+        if (tid < kWave) n_bytes += 4ull * (unsigned long long)(a_len + b_len + r_len) + 24ull;
         max_len = max(max_len, (uint32_t)(a_len + b_len));
         chain += 1;
         a_off = sh_off;
@@ -1454,13 +1412,13 @@ __global__ void __launch_bounds__(kLongThreads) k_add_huge(Dev d, int r, int32_t
         a_len = r_len;
         l = r_len ? d.pool[a_off + r_len - 1] : -1;
         __syncthreads();
+        if (l < 0 || l < minrow) break;
       }
-      if (l < 0 || l < minrow) break;
     }
     max_chain = max(max_chain, chain);
     if (dense && !failed) {  // sorted form back; the region ends all zero
       if (l >= 0) {
-        if (!huge_write_back(d, gb, summ, bits, lo, ww0, sh_minw, ((l - lo) >> 5) - ww0, &a_off, &a_cap, &a_len,
+        if (!huge_write_back(d, gb, summ, bits, lo, ww0, picks.minw, ((l - lo) >> 5) - ww0, &a_off, &a_cap, &a_len,
                              red, &sh_flag, &sh_off, &sh_cap))
           failed = true;
       } else {
@@ -1489,13 +1447,16 @@ __global__ void __launch_bounds__(kLongThreads) k_add_huge(Dev d, int r, int32_t
     }
     __syncthreads();
   }
+  max_len = (uint32_t)wave_max((int32_t)max_len);
+  if (lane_id() == 0 && n_bytes) {  // every wavefront's own pivots
+    atomicAdd(&d.stats[6], n_bytes);
+    atomicMax(&d.ctr[cw::kChain + 1], max_len);
+  }
   if (tid == 0 && n_add) {
     atomicAdd(&d.stats[0], n_add);
     atomicAdd(&d.stats[2], n_tiled);
     atomicAdd(&d.stats[5], n_add - n_tiled);
-    atomicAdd(&d.stats[6], n_bytes);
     atomicMax(&d.ctr[cw::kChain], max_chain);
-    atomicMax(&d.ctr[cw::kChain + 1], max_len);
   }
 }
 
@@ -2205,9 +2166,9 @@ class Engine : public PrebuiltTarget {
     // test hooks: smaller limits push short columns through the long-column paths
     if (const char* e = std::getenv("SSQ_TEST_SHORT_MAX")) short_max_ = std::max(2, std::min(kTile, std::atoi(e)));
     if (const char* e = std::getenv("SSQ_TEST_WINDOW_BITS"))
-      long_window_ = std::max(64, std::min(kLongBits, std::atoi(e)));
+      long_window_ = std::max(128, std::min(kLongBits, std::atoi(e) & ~127));
     if (const char* e = std::getenv("SSQ_TEST_GLOBAL_BITS"))  // small regions push columns to tiled merges
-      gspan_ = std::max(64, std::min(kHugeBits, std::atoi(e) & ~31));
+      gspan_ = std::max(128, std::min(kHugeBits, std::atoi(e) & ~127));
     if (timing_)
       for (auto& e : ev_) HIPCHK(hipEventCreate(&e));
     return SSQ_OK;
@@ -2289,7 +2250,7 @@ class Engine : public PrebuiltTarget {
     for (DevBuf* b : {&b_pool_, &b_off_, &b_len_, &b_cap_, &b_low_, &b_state_, &b_removed_, &b_flag_, &b_piv_,
                       &b_left_, &b_work_, &b_misc_, &b_U_, &b_keys_, &b_cnt_, &b_e_, &b_vs_, &b_adj_,
                       &b_hash_, &b_hd_, &b_dcol_, &b_drow_, &b_ddim_, &b_drem_, &b_scan_, &b_pmeta_, &b_prem_,
-                      &b_scrc_, &b_kbase_, &b_skey_, &b_stmp_, &b_gbits_})
+                      &b_scrc_, &b_kbase_, &b_skey_, &b_stmp_, &b_gbits_, &b_app_})
       if (b->p) (void)hipFree(b->p), b->p = nullptr, b->bytes = 0;
     if (host_ctr_) (void)hipHostFree(host_ctr_), host_ctr_ = nullptr;
     if (host_tot_) (void)hipHostFree(host_tot_), host_tot_ = nullptr;
@@ -2427,7 +2388,7 @@ class Engine : public PrebuiltTarget {
   std::string err_;
   DevBuf b_pool_, b_off_, b_len_, b_cap_, b_low_, b_state_, b_removed_, b_flag_, b_piv_, b_left_, b_work_,
       b_misc_, b_U_, b_keys_, b_cnt_, b_e_, b_vs_, b_adj_, b_hash_, b_hd_, b_dcol_, b_drow_, b_ddim_,
-      b_drem_, b_scan_, b_pmeta_, b_prem_, b_scrc_, b_kbase_, b_skey_, b_stmp_;
+      b_drem_, b_scan_, b_pmeta_, b_prem_, b_scrc_, b_kbase_, b_skey_, b_stmp_, b_app_;
   int64_t arena_hint_ = 0;
   bool no_sort_dual_ = false;  // test hook: always use the atomic anti-transpose
   bool timing_ = false;
@@ -2780,6 +2741,11 @@ int Engine::init_lists(Dev& d, int32_t maxdim, const uint8_t* hd, bool neg_known
                        ssq_stats* S) {
   const int g = grid_for(d.ncols);
   hipLaunchKernelGGL(k_lookup, dim3(g), dim3(256), 0, stream_, d, hd, neg_known ? 1 : 0);
+  uint64_t* app;
+  const int64_t app_waves = (d.n + 255) / 256;
+  if (int rc_app = ensure(b_app_, (size_t)(4 * app_waves), &app)) return rc_app;
+  d.app = (uint32_t*)app;
+  hipLaunchKernelGGL(k_apparent_bits, dim3(grid_for(app_waves * kWave)), dim3(256), 0, stream_, d.n, d.piv, app);
   int32_t* rowstat = (int32_t*)(d.ctr + cw::kRowStat);
   hipLaunchKernelGGL(k_rowstat_init, dim3(1), dim3(64), 0, stream_, rowstat);
   hipLaunchKernelGGL(k_clear_compress_stats, dim3(g), dim3(256), 0, stream_, d, rowstat, rowstat + kMaxDims);
