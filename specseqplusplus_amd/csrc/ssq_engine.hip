@@ -250,13 +250,34 @@ __global__ void k_leftone(Dev d) {
   }
 }
 
+__device__ __forceinline__ int32_t wave_max(int32_t v) {
+  for (int d = kWave / 2; d > 0; d >>= 1) v = max(v, __shfl_xor(v, d, kWave));
+  return v;
+}
+__device__ __forceinline__ int32_t wave_min(int32_t v) {
+  for (int d = kWave / 2; d > 0; d >>= 1) v = min(v, __shfl_xor(v, d, kWave));
+  return v;
+}
+
+// Extremes and counts over a whole grid.  Atomics on one address take about 11 ns each however
+// many workgroups issue them, so a workgroup combines its wavefronts' values in LDS and issues
+// one, and an extreme only where it improves on the value that is there (a relaxed load: a stale
+// one costs an atomic, no more).  With an atomic per wavefront these set the time of the passes
+// that end in them (16,384 wavefronts: 190 us for one address).
+__device__ __forceinline__ void grid_max(int32_t* p, int32_t v) {
+  if (v > __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMax(p, v);
+}
+__device__ __forceinline__ void grid_min(int32_t* p, int32_t v) {
+  if (v < __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) atomicMin(p, v);
+}
+
 // Apparent pairs and the positive-facet flag (kernel.h:459-481): the youngest facet of a
 // column is positive (its column reduces to zero; flag[row] = 1); a column that is leftmost
 // in its low row is an apparent pair; a column leftmost in any row is negative
 // (flag[n + col] = 1).  The two flags live in separate bytes: plain stores of 1 only.
 // Also collects the dimensions that hold a negative cell (one bit each, for compression).
 __global__ void k_lookup(Dev d, const uint8_t* hdclear, int neg_known) {
-  uint32_t apparent = 0;  // summed per wavefront: one atomic per wave, not per pair
+  uint32_t apparent = 0;
   uint32_t negdims = 0;
   GRID_STRIDE(c, d.ncols) {
     const int32_t l = d.len[c];
@@ -290,8 +311,17 @@ __global__ void k_lookup(Dev d, const uint8_t* hdclear, int neg_known) {
     apparent += __shfl_xor(apparent, k, kWave);
     negdims |= __shfl_xor(negdims, k, kWave);
   }
-  if (lane_id() == 0 && apparent) atomicAdd(&d.ctr[cw::kApparent], apparent);
-  if (lane_id() == 0 && negdims) atomicOr(&d.ctr[cw::kNegDims], negdims);
+  __shared__ uint32_t s_apparent, s_negdims;
+  if (threadIdx.x == 0) s_apparent = s_negdims = 0;
+  __syncthreads();
+  if (lane_id() == 0 && apparent) atomicAdd(&s_apparent, apparent);
+  if (lane_id() == 0 && negdims) atomicOr(&s_negdims, negdims);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    if (s_apparent) atomicAdd(&d.ctr[cw::kApparent], s_apparent);
+    if (s_negdims & ~__hip_atomic_load(&d.ctr[cw::kNegDims], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+      atomicOr(&d.ctr[cw::kNegDims], s_negdims);
+  }
   if (hdclear)
     GRID_STRIDE(c, d.ncols) if (hdclear[c]) d.flag[c] = 1;
 }
@@ -326,15 +356,6 @@ __global__ void k_apparent_bits(int64_t n, const uint32_t* piv, uint64_t* app) {
     }
     if (lane < 4) app[w * 4 + lane] = lane == 0 ? m[0] : lane == 1 ? m[1] : lane == 2 ? m[2] : m[3];
   }
-}
-
-__device__ __forceinline__ int32_t wave_max(int32_t v) {
-  for (int d = kWave / 2; d > 0; d >>= 1) v = max(v, __shfl_xor(v, d, kWave));
-  return v;
-}
-__device__ __forceinline__ int32_t wave_min(int32_t v) {
-  for (int d = kWave / 2; d > 0; d >>= 1) v = min(v, __shfl_xor(v, d, kWave));
-  return v;
 }
 
 // Clearing, compression and the per-dimension row bounds of the page schedule in one pass
@@ -388,12 +409,23 @@ __global__ void k_clear_compress_stats(Dev d, int32_t* maxrow, int32_t* minrow) 
         }
     }
   }
+  __shared__ int32_t s_max[kMaxDims], s_min[kMaxDims];
+  if (threadIdx.x < kMaxDims) {
+    s_max[threadIdx.x] = -1;
+    s_min[threadIdx.x] = 0x7fffffff;
+  }
+  __syncthreads();
   for (int k = 0; k < kMaxDims; k++) {
     const int32_t a = wave_max(mx[k]), b = wave_min(mn[k]);
     if (lane_id() == 0) {
-      if (a >= 0) atomicMax(&maxrow[k], a);
-      if (b != 0x7fffffff) atomicMin(&minrow[k], b);
+      if (a >= 0) atomicMax(&s_max[k], a);
+      if (b != 0x7fffffff) atomicMin(&s_min[k], b);
     }
+  }
+  __syncthreads();
+  if (threadIdx.x < kMaxDims) {
+    grid_max(&maxrow[threadIdx.x], s_max[threadIdx.x]);
+    grid_min(&minrow[threadIdx.x], s_min[threadIdx.x]);
   }
 }
 
@@ -413,7 +445,6 @@ __global__ void k_pivmeta(Dev d, int r) {
 }
 
 
-// one atomic per wavefront (a plain per-thread atomic on one address serialises millions)
 __global__ void k_maxdim(int64_t n, const int32_t* dims, int32_t* out, uint32_t* bad) {
   int32_t mx = -1, b = 0;
   // four independent loads per thread and trip: enough bytes in flight for HBM
@@ -431,11 +462,22 @@ __global__ void k_maxdim(int64_t n, const int32_t* dims, int32_t* out, uint32_t*
       else mx = max(mx, x[j]);
     }
   }
+  __shared__ int32_t s_mx, s_bad;
+  if (threadIdx.x == 0) {
+    s_mx = -1;
+    s_bad = 0;
+  }
+  __syncthreads();
   mx = wave_max(mx);
   b = wave_max(b);
   if (lane_id() == 0) {
-    if (mx >= 0) atomicMax(out, mx);
-    if (b) atomicOr(bad, 1u);
+    atomicMax(&s_mx, mx);
+    if (b) s_bad = 1;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    grid_max(out, s_mx);
+    if (s_bad) atomicOr(bad, 1u);
   }
 }
 
