@@ -437,21 +437,31 @@ __global__ void k_rc_tieapply(int64_t nt, const uint64_t* skeys, const int32_t* 
 }
 
 // ---- the two endpoint lists of every coboundary column ------------------------------------
-// One workgroup per vertex v.  For each word block w, the block stages word w of Q(m), its
-// prefix count and TB[m] for every edge m = (v, y) of v (rank order).  Column (v, z), z in the
-// block, takes the triangles {v, y, z} whose latest edge is (v, y): the y later than (v, z)
-// with z in Q((v, y)), rank TB + prefix + popcount below z.  Scanning y by rank yields them in
-// increasing rank.  v the lower endpoint: the list fills the column's foreign region from its
-// start; the higher: from its end, backwards.
-__global__ void __launch_bounds__(kBlock) k_rc_side(Grp q, const int64_t* aoff, const int32_t* inc_r,
-                                                    const uint16_t* inc_n, const uint64_t* B, const uint16_t* Bp,
-                                                    const int64_t* TB, const int32_t* rlo, const int32_t* rhi,
-                                                    const int32_t* remap, const int64_t* colptr, const int64_t* cnt,
-                                                    const int32_t* cof, int32_t* stg, int32_t* na, int32_t* nb) {
-  __shared__ uint64_t sw[kRipsMaxPoints];
-  __shared__ int32_t stb[kRipsMaxPoints];  // cloud-local TB[m], sign bit: m's run has several edges
-  __shared__ uint16_t sp[kRipsMaxPoints];
-  __shared__ int16_t zpos[kRipsMaxPoints];
+// One workgroup per vertex v.  Column (v, z) takes the triangles {v, y, z} whose latest edge is
+// (v, y): the y later than (v, z) with z in Q((v, y)), rank TB + prefix + popcount below z.
+// Scanning y by rank yields them in increasing rank.  v the lower endpoint: the list fills the
+// column's foreign region from its start; the higher: from its end, backwards.
+// The workgroup stages words of Q(m) and their prefix counts for every edge m = (v, y) of v (rank
+// order) in LDS, as many words at a time as fit, each edge's consecutive words read together: one
+// word at a time fetches every line of Q anew for each of its 16 words (20.5 ms for 40 clouds of
+// 64-2048 points; 5.7 ms this way).  A wavefront takes every kSideWaves-th neighbour z of v; its
+// lanes first load what 64 of those columns need, then the wavefront does the columns in turn.  It
+// goes over neighbours, not over all points: 24 sparse clouds of 64-4096 points 5.0 -> 0.3 ms.
+constexpr int kSideBlock = 512;
+constexpr int kSideWaves = kSideBlock / kWave;
+constexpr int kSideWords = kRipsMaxPoints;  // staged words: at least one per neighbour
+// dynamic LDS: Q words | cloud-local TB (sign bit: the run has several edges) | prefixes | neighbours
+constexpr size_t side_lds(int64_t nmax) { return (size_t)kSideWords * 10 + (size_t)nmax * 6; }
+__global__ void __launch_bounds__(kSideBlock) k_rc_side(Grp q, int nmax, const int64_t* aoff, const int32_t* inc_r,
+                                                        const uint16_t* inc_n, const uint64_t* B, const uint16_t* Bp,
+                                                        const int64_t* TB, const int32_t* rlo, const int32_t* rhi,
+                                                        const int32_t* remap, const int64_t* colptr,
+                                                        const int64_t* cnt, const int32_t* cof, int32_t* stg,
+                                                        int32_t* na, int32_t* nb) {
+  extern __shared__ uint64_t sw[];
+  int32_t* stb = (int32_t*)(sw + kSideWords);
+  uint16_t* sp = (uint16_t*)(stb + nmax);
+  uint16_t* snb = sp + kSideWords;
   const int t = threadIdx.x, lane = lane_id(), wv = t / kWave;
   const int64_t stg0 = 2 * q.NE;  // the edge columns' rows start after the vertex columns'
   for (int64_t v = blockIdx.x; v < q.NV; v += gridDim.x) {
@@ -460,54 +470,68 @@ __global__ void __launch_bounds__(kBlock) k_rc_side(Grp q, const int64_t* aoff, 
     const int W = words_of(n);
     const int64_t ao = aoff[v], e0 = q.eb[g], Eg = q.eb[g + 1] - e0, tbc = q.tb[g];
     const int deg = (int)(aoff[v + 1] - ao);
-    for (int x = t; x < n; x += kBlock) zpos[x] = -1;
-    __syncthreads();
-    for (int i = t; i < deg; i += kBlock) zpos[inc_n[ao + i]] = (int16_t)i;
-    for (int w = 0; w < W; w++) {
-      __syncthreads();
-      for (int i = t; i < deg; i += kBlock) {
-        const int64_t k = inc_r[ao + i], p = e0 + k;
-        sw[i] = B[q.bb[g] + k * W + w];
-        sp[i] = Bp[q.bb[g] + k * W + w];
-        const uint32_t tie = rhi[p] - rlo[p] > 1 ? 0x80000000u : 0u;
-        stb[i] = (int32_t)((uint32_t)(TB[p] - tbc) | tie);
-      }
-      __syncthreads();
-      for (int zz = wv; zz < 64; zz += kWaves) {
-        const int z = w * 64 + zz;
-        if (z >= n) break;
-        const int iz = zpos[z];
-        if (iz < 0) continue;
-        const int64_t kz = inc_r[ao + iz], pe = e0 + kz;
-        const int64_t cb = colptr[q.NV + e0 + (Eg - 1 - kz)] - stg0;
-        const int64_t F = cof[pe] - cnt[pe];
-        const bool lower = vl < z;
-        const uint64_t below = (1ull << zz) - 1;
-        int64_t written = 0;
-        for (int i0 = iz + 1; i0 < deg; i0 += kWave) {
-          const int i = i0 + lane;
-          bool hit = false;
-          int32_t rho = 0;
-          if (i < deg) {
-            const uint64_t x = sw[i];
-            if ((x >> zz) & 1ull) {
-              hit = true;
-              const uint32_t s = (uint32_t)stb[i];
-              rho = (int32_t)(s & 0x7fffffffu) + sp[i] + __popcll(x & below);
-              if (s & 0x80000000u) rho = remap[tbc + rho];
-            }
-          }
-          const uint64_t m = __ballot(hit);
-          if (hit) {
-            const int64_t pos = written + __popcll(m & lanes_below());
-            if (pos < F) stg[cb + (lower ? pos : F - 1 - pos)] = rho;  // more than F: reported by the merge
-          }
-          written += __popcll(m);
-        }
-        if (lane == 0) (lower ? na : nb)[pe] = (int32_t)written;
-      }
+    if (deg == 0) continue;
+    const int P = min(W, kSideWords / deg);  // words per pass
+    for (int i = t; i < deg; i += kSideBlock) {
+      const int64_t p = e0 + inc_r[ao + i];
+      const uint32_t tie = rhi[p] - rlo[p] > 1 ? 0x80000000u : 0u;
+      stb[i] = (int32_t)((uint32_t)(TB[p] - tbc) | tie);
+      snb[i] = inc_n[ao + i];
     }
-    __syncthreads();
+    for (int w0 = 0; w0 < W; w0 += P) {
+      const int pw = min(P, W - w0);
+      for (int x = t; x < deg * pw; x += kSideBlock) {
+        const int i = x / pw, w = x - i * pw;
+        const int64_t at = q.bb[g] + (int64_t)inc_r[ao + i] * W + w0 + w;
+        sw[w * deg + i] = B[at];
+        sp[w * deg + i] = Bp[at];
+      }
+      __syncthreads();
+      for (int i0 = wv; i0 < deg; i0 += kSideBlock) {
+        const int iz = i0 + lane * kSideWaves;
+        const int z = iz < deg ? snb[iz] : 0;
+        const bool in = iz < deg && (z >> 6) >= w0 && (z >> 6) < w0 + pw;
+        int64_t cb = 0, pe = 0;
+        int32_t F = 0, mine = 0;
+        if (in) {
+          const int64_t kz = inc_r[ao + iz];
+          pe = e0 + kz;
+          cb = colptr[q.NV + e0 + (Eg - 1 - kz)] - stg0;
+          F = cof[pe] - (int32_t)cnt[pe];
+        }
+        uint64_t todo = __ballot(in);
+        while (todo) {
+          const int l = __ffsll((unsigned long long)todo) - 1;
+          todo &= todo - 1;
+          const int zl = __builtin_amdgcn_readlane(z, l), Fl = __builtin_amdgcn_readlane(F, l);
+          int32_t* out = stg + ((int64_t)(uint32_t)__builtin_amdgcn_readlane((int)(cb & 0xffffffff), l) |
+                                ((int64_t)__builtin_amdgcn_readlane((int)(cb >> 32), l) << 32));
+          const uint64_t* wz = sw + ((zl >> 6) - w0) * deg;
+          const uint16_t* pz = sp + ((zl >> 6) - w0) * deg;
+          const int bit = zl & 63;
+          const uint64_t below = (1ull << bit) - 1;
+          const bool lower = vl < zl;
+          int written = 0;
+          for (int j0 = i0 + l * kSideWaves + 1; j0 < deg; j0 += kWave) {
+            const int j = j0 + lane;
+            const uint64_t x = j < deg ? wz[j] : 0ull;
+            const bool hit = (x >> bit) & 1ull;
+            const uint64_t m = __ballot(hit);
+            if (hit) {
+              const uint32_t s = (uint32_t)stb[j];
+              int32_t rho = (int32_t)(s & 0x7fffffffu) + pz[j] + __popcll(x & below);
+              if (s & 0x80000000u) rho = remap[tbc + rho];
+              const int pos = written + __popcll(m & lanes_below());
+              if (pos < Fl) out[lower ? pos : Fl - 1 - pos] = rho;  // more than F: reported by the merge
+            }
+            written += __popcll(m);
+          }
+          if (lane == l) mine = written;
+        }
+        if (in) (vl < z ? na : nb)[pe] = mine;
+      }
+      __syncthreads();
+    }
   }
 }
 
@@ -523,25 +547,22 @@ __global__ void __launch_bounds__(kBlock) k_rc_side(Grp q, const int64_t* aoff, 
 __device__ __forceinline__ int32_t own_rank(const int32_t* remap, bool tie, int64_t base, int64_t own0, int i) {
   return tie ? remap[base + own0 + i] : (int32_t)(own0 + i);
 }
-// number of entries > x in an ascending list / a descending list / the own list
-__device__ __forceinline__ int count_gt_asc(const int32_t* v, int n, int32_t x) {
-  int lo = 0, hi = n;  // first index with v > x
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (v[mid] <= x) lo = mid + 1;
-    else hi = mid;
+// For each of U values: how many entries of the list v (ascending or descending) are larger.  The
+// U searches go step by step together, so their reads overlap.
+template <bool kAsc, int U>
+__device__ __forceinline__ void count_gt(const int32_t* v, int n, const int32_t (&x)[U], int (&c)[U]) {
+  int lo[U] = {};
+  for (int s = n > 0 ? 1 << (31 - __clz(n)) : 0; s > 0; s >>= 1) {
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int k = lo[u] + s;
+      if (k <= n && (kAsc ? v[k - 1] <= x[u] : v[k - 1] > x[u])) lo[u] = k;
+    }
   }
-  return n - lo;
+#pragma unroll
+  for (int u = 0; u < U; u++) c[u] = kAsc ? n - lo[u] : lo[u];
 }
-__device__ __forceinline__ int count_gt_desc(const int32_t* v, int n, int32_t x) {
-  int lo = 0, hi = n;  // first index with v < x (v > x before it)
-  while (lo < hi) {
-    const int mid = (lo + hi) >> 1;
-    if (v[mid] > x) lo = mid + 1;
-    else hi = mid;
-  }
-  return lo;
-}
+// ... and in the own list
 __device__ __forceinline__ int count_gt_own(const int32_t* remap, bool tie, int64_t base, int64_t own0, int n,
                                             int32_t x) {
   if (!tie) {  // own0 .. own0 + n - 1
@@ -557,51 +578,145 @@ __device__ __forceinline__ int count_gt_own(const int32_t* remap, bool tie, int6
   return n - lo;
 }
 
-__global__ void __launch_bounds__(kBlock) k_rc_merge(Grp q, const int32_t* ecl, const int32_t* rlo, const int32_t* rhi,
-                                                     const int64_t* TB, const int32_t* remap, const int64_t* colptr,
-                                                     const int64_t* cnt, const int32_t* cof, const int32_t* na,
-                                                     const int32_t* nb, const int32_t* stg, int32_t* pool,
-                                                     uint32_t* leftone, uint32_t* err) {
-  const int lane = lane_id(), wv = threadIdx.x / kWave;
-  const int64_t stg0 = 2 * q.NE;
-  for (int64_t p = (int64_t)blockIdx.x * kWaves + wv; p < q.NE; p += (int64_t)gridDim.x * kWaves) {
-    const int g = ecl[p];
-    const int64_t e0 = q.eb[g], k = p - e0, tbc = q.tb[g];
-    const int64_t col = edid(q, g, k);
-    const int64_t c0 = colptr[col];
-    const int32_t len = cof[p], own = (int32_t)cnt[p], F = len - own;
-    const int32_t an = na[p], bn = nb[p];
-    if (an + bn != F || an < 0 || bn < 0 || own < 0) {
-      if (lane == 0) atomicOr(err, 1u);
-      continue;
-    }
-    const bool tie = own > 0 && rhi[p] - rlo[p] > 1;
-    const int32_t* Aa = stg + (c0 - stg0);  // ascending, an entries
-    const int32_t* Bd = Aa + (F - bn);      // descending, bn entries
-    int32_t* out = pool + c0;
-    const int64_t own0 = TB[p] - tbc;
-    for (int i = lane; i < an; i += kWave) {
-      const int32_t x = Aa[i];
-      const int pos = (an - 1 - i) + count_gt_desc(Bd, bn, x) + count_gt_own(remap, tie, tbc, own0, own, x);
-      out[pos] = (int32_t)tdid(q, g, x);
-    }
-    for (int j = lane; j < bn; j += kWave) {
-      const int32_t y = Bd[j];
-      const int pos = j + count_gt_asc(Aa, an, y) + count_gt_own(remap, tie, tbc, own0, own, y);
-      out[pos] = (int32_t)tdid(q, g, y);
-    }
+// One column by one wavefront.  L: its foreign entries (an ascending, then bn descending), in LDS
+// or in device memory.  The merged column is put together in LDS, kMergeOut entries at a time, and
+// leaves it in order, checked on the way (strictly increasing, below n).  Without a tie every
+// foreign triangle is later than the own ones.  Returns whether the check failed.
+constexpr int kMergeIn = 1024, kMergeOut = 1024, kMergeU = 2;
+__device__ __forceinline__ bool merge_column(const int32_t* L, int an, int bn, int own, int64_t own0, bool tie,
+                                             const int32_t* remap, int64_t tbc, int64_t last, int64_t n,
+                                             uint32_t col, int32_t* sout, int32_t* out, uint32_t* leftone) {
+  const int lane = lane_id(), F = an + bn, len = F + own;
+  const int32_t* Bd = L + an;
+  bool bad = false;
+  int32_t before = -1;
+  for (int o0 = 0; o0 < len; o0 += kMergeOut) {
+    const int m = min(kMergeOut, len - o0);
+    // foreign entries k, k + 64, ... below end, all of one list: after the larger ones of both lists
+    const auto place = [&](int k, int end) {
+      int32_t x[kMergeU];
+      int c[kMergeU];
+#pragma unroll
+      for (int u = 0; u < kMergeU; u++) x[u] = k + u * kWave < end ? L[k + u * kWave] : 0;
+      if (end == F && k >= an) count_gt<true>(L, an, x, c);
+      else count_gt<false>(Bd, bn, x, c);
+#pragma unroll
+      for (int u = 0; u < kMergeU; u++) {
+        const int i = k + u * kWave;
+        if (i >= end) break;
+        int pos = c[u] + (i >= an ? i - an : an - 1 - i) - o0;
+        if (tie) pos += count_gt_own(remap, tie, tbc, own0, own, x[u]);
+        if (pos >= 0 && pos < m) sout[pos] = (int32_t)(last - x[u]);
+      }
+    };
+    for (int i = lane; i < an; i += kWave * kMergeU) place(i, an);
+    for (int j = lane; j < bn; j += kWave * kMergeU) place(an + j, F);
     for (int i = lane; i < own; i += kWave) {
       const int32_t z = own_rank(remap, tie, tbc, own0, i);
-      const int pos = (own - 1 - i) + count_gt_asc(Aa, an, z) + count_gt_desc(Bd, bn, z);
-      const int64_t d = tdid(q, g, z);
-      out[pos] = (int32_t)d;
-      leftone[d] = (uint32_t)col;
+      int pos = own - 1 - i - o0;
+      if (tie) {
+        const int32_t zz[1] = {z};
+        int ca[1], cb[1];
+        count_gt<true>(L, an, zz, ca);
+        count_gt<false>(Bd, bn, zz, cb);
+        pos += ca[0] + cb[0];
+      } else {
+        pos += F;
+      }
+      if (pos >= 0 && pos < m) {
+        sout[pos] = (int32_t)(last - z);
+        leftone[last - z] = col;
+      }
     }
+    wave_sync();
+    for (int i = lane; i < m; i += kWave) {
+      const int32_t x = sout[i], prev = i > 0 ? sout[i - 1] : before;
+      bad |= x <= prev || x >= n;
+      out[o0 + i] = x;
+    }
+    before = sout[m - 1];
+    wave_sync();
+  }
+  return bad;
+}
+
+// A wavefront takes `batch` (at most 64) consecutive columns: its lanes load what each of them
+// needs (three dependent gathers, once for all), and the foreign list of a column is on its way to
+// registers while the column before it is merged.  The list goes through LDS if it fits: the
+// searches' scattered reads stay on chip.  One column at a time, with the lists searched in device
+// memory and the entries written where they fall, took 13.2 ms for 40 clouds of 64-2048 points
+// (8.7e8 entries), and the check 2.6 ms in a pass of its own; now 6.2 ms.
+__global__ void __launch_bounds__(kBlock) k_rc_merge(Grp q, int batch, const int32_t* ecl, const int32_t* rlo,
+                                                     const int32_t* rhi, const int64_t* TB, const int32_t* remap,
+                                                     const int64_t* colptr, const int64_t* cnt, const int32_t* cof,
+                                                     const int32_t* na, const int32_t* nb, const int32_t* stg,
+                                                     int32_t* pool, uint32_t* leftone, uint32_t* err) {
+  __shared__ int32_t s_in[kWaves][kMergeIn], s_out[kWaves][kMergeOut];
+  const int lane = lane_id(), wv = threadIdx.x / kWave;
+  const int64_t stg0 = 2 * q.NE, n = q.NV + q.NE + q.NT;
+  constexpr int kAhead = 8;  // registers of a list loaded ahead: its first 512 entries
+  for (int64_t p0 = ((int64_t)blockIdx.x * kWaves + wv) * batch; p0 < q.NE; p0 += (int64_t)gridDim.x * kWaves * batch) {
+    const int64_t p = p0 + lane;
+    int64_t c0 = 0, own0 = 0, tbc = 0, last = 0, col = 0;
+    int32_t own = 0, an = 0, bn = 0;
+    bool tie = false, ok = false, bad = false;
+    if (lane < batch && p < q.NE) {
+      const int g = ecl[p];
+      tbc = q.tb[g];
+      col = edid(q, g, p - q.eb[g]);
+      c0 = colptr[col];
+      own = (int32_t)cnt[p];
+      an = na[p];
+      bn = nb[p];
+      ok = an >= 0 && bn >= 0 && own >= 0 && an + bn + own == cof[p];
+      bad = !ok;
+      tie = own > 0 && rhi[p] - rlo[p] > 1;
+      own0 = TB[p] - tbc;
+      last = tdid(q, g, 0);  // the dual id falls as the rank grows
+    }
+    if (__ballot(bad) && lane == 0) atomicOr(err, 1u);
+    bad = false;
+    const auto at = [](int64_t x, int l) {
+      return (int64_t)(uint32_t)__builtin_amdgcn_readlane((int)(x & 0xffffffff), l) |
+             ((int64_t)__builtin_amdgcn_readlane((int)(x >> 32), l) << 32);
+    };
+    int32_t r[kAhead];
+    const auto ahead = [&](int l) {
+      const int32_t F = __builtin_amdgcn_readlane(an + bn, l);
+      const int32_t* lists = stg + (at(c0, l) - stg0);
+#pragma unroll
+      for (int u = 0; u < kAhead; u++) r[u] = lane + u * kWave < F ? lists[lane + u * kWave] : 0;
+    };
+    uint64_t todo = __ballot(ok);
+    if (todo) ahead(__ffsll((unsigned long long)todo) - 1);
+    while (todo) {
+      const int l = __ffsll((unsigned long long)todo) - 1;
+      todo &= todo - 1;
+      const int32_t a = __builtin_amdgcn_readlane(an, l), b = __builtin_amdgcn_readlane(bn, l), F = a + b;
+      const int32_t o = __builtin_amdgcn_readlane(own, l);
+      const bool t = __builtin_amdgcn_readlane((int)tie, l) != 0;
+      const int64_t base = at(c0, l), o0 = at(own0, l), tb = at(tbc, l), la = at(last, l);
+      const uint32_t cl = (uint32_t)__builtin_amdgcn_readlane((int)col, l);
+      const int32_t* lists = stg + (base - stg0);
+      if (F <= kMergeIn) {
+#pragma unroll
+        for (int u = 0; u < kAhead; u++)
+          if (lane + u * kWave < F) s_in[wv][lane + u * kWave] = r[u];
+        for (int i = kAhead * kWave + lane; i < F; i += kWave) s_in[wv][i] = lists[i];
+        wave_sync();
+        if (todo) ahead(__ffsll((unsigned long long)todo) - 1);
+        bad |= merge_column(s_in[wv], a, b, o, o0, t, remap, tb, la, n, cl, s_out[wv], pool + base, leftone);
+      } else {
+        if (todo) ahead(__ffsll((unsigned long long)todo) - 1);
+        bad |= merge_column(lists, a, b, o, o0, t, remap, tb, la, n, cl, s_out[wv], pool + base, leftone);
+      }
+    }
+    if (__ballot(bad) && lane == 0) atomicOr(err, 2u);
   }
 }
 
-// Every column's rows strictly increasing and below n (the engine indexes its tables with
-// them): a check of the built matrix before the reduction reads it.  One wavefront per column.
+// The rows of the first nc columns (the vertices') strictly increasing and below n, as the merge
+// checks the others': the engine indexes its tables with them.  One wavefront per column.
 __global__ void __launch_bounds__(kBlock) k_rc_check(int64_t nc, int64_t n, const int64_t* colptr, const int32_t* pool,
                                                      uint32_t* err) {
   const int lane = lane_id(), wv = threadIdx.x / kWave;
@@ -705,13 +820,15 @@ __global__ void k_rc_gather(Grp q, int pdim, const int64_t* srcv, const int64_t*
 }
 
 // Pairs from per-cloud slots to their packed place: cloud c's cnt[c] pairs move from slot[c]
-// to off[c].  One workgroup per cloud.
+// to off[c].  gridDim.y workgroups per cloud (one alone copies about 40 GB/s: 40 clouds with 61 MB
+// of pairs took 1.5 ms).
 __global__ void k_rc_pack(int C, const int64_t* slot, const int64_t* off, const int64_t* stage, int64_t* out) {
   for (int c = blockIdx.x; c < C; c += gridDim.x) {
     const int64_t n = 2 * (off[c + 1] - off[c]);
     const int64_t* src = stage + 2 * slot[c];
     int64_t* dst = out + 2 * off[c];
-    for (int64_t i = threadIdx.x; i < n; i += blockDim.x) dst[i] = src[i];
+    for (int64_t i = (int64_t)blockIdx.y * blockDim.x + threadIdx.x; i < n; i += (int64_t)gridDim.y * blockDim.x)
+      dst[i] = src[i];
   }
 }
 
@@ -1161,21 +1278,26 @@ static int rc_group(RipsCo* B, const RipsCo* S, PrebuiltTarget* eng, hipStream_t
   RCGROW(nb, int32_t, MAXE, nb);
   uint32_t* derr;
   RCGROW(err, uint32_t, 4, derr);
-  RCCHK(hipMemsetAsync(na, 0, sizeof(int32_t) * MAXE, s));
-  RCCHK(hipMemsetAsync(nb, 0, sizeof(int32_t) * MAXE, s));
   RCCHK(hipMemsetAsync(derr, 0, sizeof(uint32_t), s));
   if (NE > 0) {
-    hipLaunchKernelGGL(k_rc_side, dim3((unsigned)std::min<int64_t>(NV, 65536)), dim3(kBlock), 0, s, q,
+    int64_t nmax = 0;
+    for (int g = 0; g < G; g++) nmax = std::max(nmax, pb[g + 1] - pb[g]);
+    nmax = (nmax + 1) & ~(int64_t)1;  // the 2-byte tables behind the 4-byte one stay aligned
+    hipLaunchKernelGGL(k_rc_side, dim3((unsigned)std::min<int64_t>(NV, 65536)), dim3(kSideBlock), side_lds(nmax), s, q,
+                       (int)nmax,
                        (const int64_t*)aoff, (const int32_t*)inc_r, (const uint16_t*)inc_n, (const uint64_t*)Bq,
                        (const uint16_t*)Bp, (const int64_t*)TB, (const int32_t*)rlo, (const int32_t*)rhi,
                        (const int32_t*)remap, (const int64_t*)colptr, (const int64_t*)cnt, (const int32_t*)cof, stg,
                        na, nb);
-    hipLaunchKernelGGL(k_rc_merge, dim3(grid_of(NE, kWaves)), dim3(kBlock), 0, s, q, (const int32_t*)ecl,
+    // columns per wavefront: enough for the loads to overlap, few enough to fill the chip
+    const int batch = (int)std::max<int64_t>(1, std::min<int64_t>(kWave, NE / 8192));
+    hipLaunchKernelGGL(k_rc_merge, dim3(grid_of((NE + batch - 1) / batch, kWaves)), dim3(kBlock), 0, s, q, batch,
+                       (const int32_t*)ecl,
                        (const int32_t*)rlo, (const int32_t*)rhi, (const int64_t*)TB, (const int32_t*)remap,
                        (const int64_t*)colptr, (const int64_t*)cnt, (const int32_t*)cof, (const int32_t*)na,
                        (const int32_t*)nb, (const int32_t*)stg, pool, leftone, derr);
   }
-  hipLaunchKernelGGL(k_rc_check, dim3(grid_of(NC, kWaves)), dim3(kBlock), 0, s, NC, N, (const int64_t*)colptr,
+  hipLaunchKernelGGL(k_rc_check, dim3(grid_of(NV, kWaves)), dim3(kBlock), 0, s, NV, N, (const int64_t*)colptr,
                      (const int32_t*)pool, derr);
   RCCHK(hipGetLastError());
   RCCHK(hipMemcpyAsync(&B->host[4], derr, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
@@ -1377,7 +1499,8 @@ int ripsco_reduce(RipsCo* const* Bs, PrebuiltTarget* const* engs, int nstreams, 
   for (int c = 0; c < count; c++) pair_off[c + 1] = pair_off[c] + counts[(size_t)c];
   RCCHK(hipMemcpyAsync(dslot, slot.data(), sizeof(int64_t) * (count + 1), hipMemcpyHostToDevice, s));
   RCCHK(hipMemcpyAsync(doff, pair_off, sizeof(int64_t) * (count + 1), hipMemcpyHostToDevice, s));
-  hipLaunchKernelGGL(k_rc_pack, dim3((unsigned)std::min(count, 4096)), dim3(kBlock), 0, s, count,
+  const unsigned per = (unsigned)std::max<int64_t>(1, std::min<int64_t>(64, 2 * need / count / kBlock));
+  hipLaunchKernelGGL(k_rc_pack, dim3((unsigned)std::min(count, 4096), per), dim3(kBlock), 0, s, count,
                      (const int64_t*)dslot, (const int64_t*)doff, (const int64_t*)stage, d_pairs);
   RCCHK(hipGetLastError());
   RCCHK(hipStreamSynchronize(s));
