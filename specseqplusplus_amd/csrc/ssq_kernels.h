@@ -19,6 +19,13 @@ __device__ __forceinline__ void wave_sync() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// A value that is the same in every lane, in a scalar register: branches and loops on it are
+// scalar instead of masked.
+__device__ __forceinline__ int32_t uniform(int32_t v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ int64_t uniform64(int64_t v) {
+  return (int64_t)(uint32_t)uniform((int32_t)(v & 0xffffffff)) | ((int64_t)uniform((int32_t)(v >> 32)) << 32);
+}
+
 __device__ __forceinline__ int wave_incl_scan(int v) {
   const int lane = lane_id();
 #pragma unroll
