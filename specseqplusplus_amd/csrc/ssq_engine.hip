@@ -1120,6 +1120,74 @@ __device__ __forceinline__ void toggle_rows(const int32_t* B, int32_t len, int t
   }
 }
 
+// Every set bit of the words [w0, w1) of a source, in order: each wavefront takes a contiguous part,
+// 256 words (eight chunks) at a time, four of them in flight, a uint4 per lane.  get(w) returns
+// the four words at w (w a multiple of 4), skip(w) whether the 256 words at w are known to be zero.
+// count_bits returns this thread's bits; emit_bits writes the rows of this wavefront's part to O
+// from `pos` (the wavefront's first position) on.
+constexpr int kGroupWords = 4 * kWave;
+struct WaveSpan {
+  int32_t w0, w1;
+};
+__device__ __forceinline__ WaveSpan wave_span(int32_t w0, int32_t w1) {
+  const int32_t groups = w1 > w0 ? (w1 - w0 + kGroupWords - 1) / kGroupWords : 0;
+  const int32_t per = (groups + kLongThreads / kWave - 1) / (kLongThreads / kWave);
+  const int32_t a = w0 + (int32_t)(threadIdx.x / kWave) * per * kGroupWords;
+  return {min(a, w1), min(a + per * kGroupWords, w1)};
+}
+template <typename GetF, typename SkipF>
+__device__ __forceinline__ int32_t count_bits(int32_t w0, int32_t w1, GetF get, SkipF skip) {
+  const WaveSpan sp = wave_span(w0, w1);
+  int32_t n = 0;
+  for (int32_t w = sp.w0; w < sp.w1; w += 4 * kGroupWords) {
+    uint4 v[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int32_t g = w + u * kGroupWords, x = g + 4 * lane_id();
+      v[u] = make_uint4(0u, 0u, 0u, 0u);
+      if (g < sp.w1 && !skip(g) && x < w1) v[u] = get(x);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++) n += __popc(v[u].x) + __popc(v[u].y) + __popc(v[u].z) + __popc(v[u].w);
+  }
+  return n;
+}
+template <typename GetF, typename SkipF, typename ClearF>
+__device__ __forceinline__ void emit_bits(int32_t w0, int32_t w1, GetF get, SkipF skip, ClearF clear, int32_t row0,
+                                          int32_t* O, int32_t pos) {
+  const WaveSpan sp = wave_span(w0, w1);
+  for (int32_t w = sp.w0; w < sp.w1; w += 4 * kGroupWords) {
+    uint4 v[4];
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int32_t g = w + u * kGroupWords, x = g + 4 * lane_id();
+      v[u] = make_uint4(0u, 0u, 0u, 0u);
+      if (g < sp.w1 && !skip(g) && x < w1) v[u] = get(x);
+    }
+#pragma unroll
+    for (int u = 0; u < 4; u++) {
+      const int32_t n = __popc(v[u].x) + __popc(v[u].y) + __popc(v[u].z) + __popc(v[u].w);
+      if (!__ballot(n > 0)) continue;
+      const int32_t x = w + u * kGroupWords + 4 * lane_id();
+      if (n > 0) clear(x);
+      const int32_t incl = wave_incl_scan(n);
+      if (O) {
+        int32_t at = pos + incl - n;
+        const uint32_t ws[4] = {v[u].x, v[u].y, v[u].z, v[u].w};
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+          uint32_t m = ws[j];
+          while (m) {
+            O[at++] = row0 + ((x + j) << 5) + __ffs(m) - 1;
+            m &= m - 1;
+          }
+        }
+      }
+      pos += __shfl(incl, kWave - 1, kWave);
+    }
+  }
+}
+
 __global__ void __launch_bounds__(kLongThreads) k_add_long(Dev d, int r, int32_t minrow) {
   __shared__ __align__(16) uint32_t bits[kLongWords];
   __shared__ Picks picks;
@@ -1201,12 +1269,10 @@ __global__ void __launch_bounds__(kLongThreads) k_add_long(Dev d, int r, int32_t
       max_chain = max(max_chain, chain);
       // the bit set back in sorted form
       const int32_t W = l >= 0 ? ((l - lo) >> 5) + 1 : 0;
+      const auto window = [&](int32_t w) { return *(const uint4*)(bits + w); };
+      const auto never = [](int32_t) { return false; };
       int32_t total;
-      const int32_t per = (W + kLongThreads - 1) / kLongThreads;
-      const int32_t w0 = min(W, tid * per), w1 = min(W, w0 + per);
-      int32_t pc = 0;
-      for (int32_t w = w0; w < w1; w++) pc += __popc(bits[w]);
-      const int32_t pos0 = block_excl_scan(pc, red, &total);
+      const int32_t pos0 = __shfl(block_excl_scan(count_bits(0, W, window, never), red, &total), 0, kWave);
       if (tid == 0) {
         int64_t o = a_off;
         int32_t cp = a_cap;
@@ -1220,16 +1286,7 @@ __global__ void __launch_bounds__(kLongThreads) k_add_long(Dev d, int r, int32_t
       else {
         a_off = sh_off;
         a_cap = sh_cap;
-        int32_t* O = d.pool + a_off;
-        int32_t pos = pos0;
-        for (int32_t w = w0; w < w1; w++) {
-          uint32_t x = bits[w];
-          while (x) {
-            const int b = __ffs(x) - 1;
-            O[pos++] = lo + (w << 5) + b;
-            x &= x - 1;
-          }
-        }
+        emit_bits(0, W, window, never, [](int32_t) {}, lo, d.pool + a_off, pos0);
         a_len = total;
       }
     }
@@ -1337,34 +1394,28 @@ __device__ __forceinline__ int32_t tail_top(uint32_t* summ, const uint32_t* gb, 
   return -1;
 }
 
-// The column back in sorted form: the tail's marked chunks of region words [w_lo, ww0) (each
-// word read is cleared), then the window's words up to LDS word top_w.  Returns false when the
-// store is exhausted (the region is cleared all the same).
+// The column back in sorted form: the tail's marked chunks of region words [w_lo, ww0) (each word
+// read is cleared), then the window's words up to LDS word top_w.  Returns false when the store is
+// exhausted (the region is cleared all the same).  A thread per chunk, word by word, took 2.5 ms
+// for a column of 280,000 rows over 35 M (a third of k_add_huge on a dense Rips cloud), 1.7 ms
+// with the words read 1 KB at a time.
 __device__ bool huge_write_back(Dev& d, uint32_t* gb, const uint32_t* summ, const uint32_t* bits, int32_t lo,
                                 int32_t ww0, int32_t w_lo, int32_t top_w, int64_t* a_off, int32_t* a_cap,
                                 int32_t* a_len, int32_t* red, int32_t* sh_flag, int64_t* sh_off, int32_t* sh_cap) {
   const int tid = threadIdx.x;
-  const int32_t nwords = d.gspan >> 5;
-  __threadfence();  // the last addition's global toggles, before the tail is read
+  __threadfence();  // the last addition's global toggles, before the tail is read (plain loads below)
   __syncthreads();
-  // tail chunks [c_lo, c_hi] (ww0 is chunk-aligned: the tail ends at a chunk boundary)
-  const int32_t c_lo = max(w_lo, 0) >> 5, c_hi = (ww0 >> 5) - 1;
-  const int32_t C = c_hi >= c_lo ? c_hi - c_lo + 1 : 0;
-  const int32_t per = (C + kLongThreads - 1) / kLongThreads;
-  const int32_t v0 = c_lo + min(C, tid * per), v1 = c_lo + min(C, tid * per + per);
-  const int32_t WW = top_w >= 0 ? top_w + 1 : 0;  // window words in use
-  const int32_t wper = (WW + kLongThreads - 1) / kLongThreads;
-  const int32_t u0 = min(WW, tid * wper), u1 = min(WW, tid * wper + wper);
-  int32_t pt = 0, pw = 0;
-  for (int32_t ch = v0; ch < v1; ch++) {
-    if (!chunk_marked(summ, ch)) continue;
-    const int32_t ke = min(kChunkWords, nwords - (ch << 5));
-    for (int32_t k = 0; k < ke; k++) pt += __popc(gload(gb + (ch << 5) + k));
-  }
-  for (int32_t w = u0; w < u1; w++) pw += __popc(bits[w]);
+  const int32_t t0 = max(w_lo, 0) & ~(kGroupWords - 1), t1 = ww0;  // tail words (ww0 is chunk-aligned)
+  const int32_t WW = top_w >= 0 ? top_w + 1 : 0;                   // window words in use
+  const auto tail = [&](int32_t w) { return *(const uint4*)(gb + w); };
+  const auto unmarked = [&](int32_t w) { return ((summ[w >> 10] >> ((w >> 5) & 24)) & 0xffu) == 0u; };
+  const auto window = [&](int32_t w) { return *(const uint4*)(bits + w); };
+  const auto never = [](int32_t) { return false; };
   int32_t total_t, total_w;
-  const int32_t post = block_excl_scan(pt, red, &total_t);
-  const int32_t posw = block_excl_scan(pw, red, &total_w);
+  int32_t post = block_excl_scan(count_bits(t0, t1, tail, unmarked), red, &total_t);
+  int32_t posw = block_excl_scan(count_bits(0, WW, window, never), red, &total_w);
+  post = __shfl(post, 0, kWave);  // the wavefront's first position
+  posw = __shfl(posw, 0, kWave);
   const int32_t total = total_t + total_w;
   if (tid == 0) {
     int64_t o = *a_off;
@@ -1376,35 +1427,9 @@ __device__ bool huge_write_back(Dev& d, uint32_t* gb, const uint32_t* summ, cons
   }
   __syncthreads();
   const bool ok = *sh_flag != 0;
-  int32_t* O = d.pool + *sh_off;
-  int32_t pos = post;
-  for (int32_t ch = v0; ch < v1; ch++) {
-    if (!chunk_marked(summ, ch)) continue;
-    const int32_t ke = min(kChunkWords, nwords - (ch << 5));
-    for (int32_t k = 0; k < ke; k++) {
-      const int32_t g = (ch << 5) + k;
-      uint32_t x = gload(gb + g);
-      if (!x) continue;
-      gb[g] = 0u;
-      if (ok)
-        while (x) {
-          const int b = __ffs(x) - 1;
-          O[pos++] = lo + (g << 5) + b;
-          x &= x - 1;
-        }
-    }
-  }
-  pos = total_t + posw;
-  const int32_t wrow0 = lo + (ww0 << 5);
-  if (ok)
-    for (int32_t w = u0; w < u1; w++) {
-      uint32_t x = bits[w];
-      while (x) {
-        const int b = __ffs(x) - 1;
-        O[pos++] = wrow0 + (w << 5) + b;
-        x &= x - 1;
-      }
-    }
+  int32_t* O = ok ? d.pool + *sh_off : nullptr;
+  emit_bits(t0, t1, tail, unmarked, [&](int32_t w) { *(uint4*)(gb + w) = make_uint4(0u, 0u, 0u, 0u); }, lo, O, post);
+  if (ok) emit_bits(0, WW, window, never, [](int32_t) {}, lo + (ww0 << 5), O, total_t + posw);
   __threadfence();
   __syncthreads();
   if (ok) {
@@ -1510,18 +1535,15 @@ __global__ void __launch_bounds__(kLongThreads) k_add_huge(Dev d, int r, int32_t
           if (l < 0) break;
           const int32_t lw = (l - lo) >> 5;
           const int32_t nb = window_base(lw);  // chunk-aligned, below the old window
-          // pull the marked chunks [nb >> 5, lw >> 5] into the (all zero) window
+          // pull the marked chunks [nb >> 5, lw >> 5] into the (all zero) window, a uint4 per
+          // thread (plain loads: after the fence above)
           const int32_t c0 = nb >> 5, C = (lw >> 5) - c0 + 1;
-          for (int32_t ci = tid; ci < C; ci += kLongThreads) {
-            const int32_t ch = c0 + ci;
-            if (!chunk_marked(summ, ch)) continue;
-            const int32_t ke = min(kChunkWords, nwords - (ch << 5));
-            for (int32_t k = 0; k < ke; k++) {
-              const int32_t g = (ch << 5) + k;
-              const uint32_t x = gload(gb + g);
-              bits[g - nb] = x;
-              if (x) gb[g] = 0u;
-            }
+          for (int32_t k = tid; k < C * (kChunkWords / 4); k += kLongThreads) {
+            const int32_t g = nb + 4 * k;
+            if (g >= nwords || !chunk_marked(summ, g >> 5)) continue;
+            const uint4 x = *(const uint4*)(gb + g);
+            *(uint4*)(bits + g - nb) = x;
+            if (x.x | x.y | x.z | x.w) *(uint4*)(gb + g) = make_uint4(0u, 0u, 0u, 0u);
           }
           __syncthreads();
           for (int32_t ci = tid; ci < C; ci += kLongThreads) {  // every pulled chunk is now zero
