@@ -42,6 +42,7 @@
 
 #include "ssq_internal.h"
 #include "ssq_kernels.h"
+#include "ssq_sort.h"
 
 namespace ssq {
 
@@ -432,20 +433,21 @@ __global__ void k_clear_compress_stats(Dev d, int32_t* maxrow, int32_t* minrow) 
 }
 
 // After a claim round: the winners publish where their columns are stored.
-__global__ void k_pivmeta(Dev d, int r) {
+__device__ __forceinline__ void publish_pivots(const Dev& d, int r) {
   const int in = r & 1;
   const uint32_t cnt = d.ctr[cw::kW + in];
   const int32_t* list = d.work[in];
   for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < cnt; i += (int64_t)gridDim.x * blockDim.x) {
     const int32_t c = list[i];
     const int32_t l = d.low[c];
-    if (d.piv[l] == (uint32_t)c) {
+    // past the L1, which may hold the entry as it was before this launch's claims
+    if (__hip_atomic_load(&d.piv[l], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (uint32_t)c) {
       const int64_t o = d.off[c];
       d.pivmeta[l] = pivmeta_of(o, d.len[c], d.pool + o);
     }
   }
 }
-
+__global__ void k_pivmeta(Dev d, int r) { publish_pivots(d, r); }
 
 __global__ void k_maxdim(int64_t n, const int32_t* dims, int32_t* out, uint32_t* bad) {
   int32_t mx = -1, b = 0;
@@ -576,7 +578,7 @@ __global__ void k_scan_window(Dev d, const int32_t* cols, int32_t ncols, int32_t
 }
 
 // Claim round r: pivot claims by atomicMin on the pivot table (kernel.h:583-607).
-__global__ void k_claim(Dev d, int r) {
+__device__ __forceinline__ void claim_pivots(const Dev& d, int r) {
   const int in = r & 1, nx = (r + 1) & 1;
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     d.ctr[cw::kA + nx] = 0;
@@ -608,7 +610,16 @@ __global__ void k_claim(Dev d, int r) {
     wave_push(add, who, d.work[2 + in], &d.ctr[cw::kA + in]);
   }
 }
-
+__global__ void k_claim(Dev d, int r) { claim_pivots(d, r); }
+// Both for a worklist of at most kOneClaim columns, by one workgroup: one launch less in each
+// round, 4.3 us for the two on short lists.  Two trips of 1024 threads are still latency (an
+// atomic and two loads each); longer lists fill the grid of the two kernels.
+constexpr int64_t kOneClaim = 2048;
+__global__ void __launch_bounds__(1024) k_claim_publish(Dev d, int r) {
+  claim_pivots(d, r);
+  __syncthreads();  // every claim's atomicMin has returned
+  publish_pivots(d, r);
+}
 
 // One wavefront: O = A xor B for sorted sets in HBM, merged kTile merged positions at a
 // time through the wave's LDS staging buffers.  Returns |O|.  O must hold |A|+|B|.
@@ -2861,6 +2872,10 @@ int Engine::guided_clear(Dev& d, int64_t n, int32_t maxdim, const int32_t* d_dim
 
 
 int Engine::scan_counts(const int32_t* cnt, int64_t n, int64_t* out) {
+  if (n <= ssq_sort::kOneScan) {  // one launch for three
+    HIPCHK((ssq_sort::scan<int32_t, int64_t, false>(cnt, n, out, nullptr, stream_)));
+    return SSQ_OK;
+  }
   const int64_t nb = std::max<int64_t>(1, (n + kScanTile - 1) / kScanTile);
   int64_t* bsum;
   int rc = ensure(b_scan_, (size_t)(nb + 1), &bsum);
@@ -3031,9 +3046,9 @@ int Engine::page_loop(Dev& d, const ssq_params& p, int32_t maxdim, const LoopPla
   const int wpg = p.add_waves > 0 ? p.add_waves : kAddWavesDefault;  // 2, 4 or 8 (checked)
   const int wsel = wpg == 2 ? 0 : wpg == 4 ? 1 : 2;
   const int add_waves = (int)std::min<int64_t>(p.queue_size, (int64_t)cus_ * add_waves_per_cu_[wsel]);
-  const int add_grid = std::max(1, (add_waves + wpg - 1) / wpg);
+  const int add_grid_max = std::max(1, (add_waves + wpg - 1) / wpg);
   const int rounds_per_sync = p.rounds_per_sync > 0 ? p.rounds_per_sync : rounds_per_sync_;
-  const int long_grid = p.long_grid > 0 ? p.long_grid : cus_ * 2;
+  const int long_grid_max = p.long_grid > 0 ? p.long_grid : cus_ * 2;
   if (p.short_max > 0) d.short_max = std::min(p.short_max, (int32_t)kTile);
   bool oom = false;
   *oom_out = false;
@@ -3052,12 +3067,24 @@ int Engine::page_loop(Dev& d, const ssq_params& p, int32_t maxdim, const LoopPla
         const int32_t fl = (int32_t)std::max<int64_t>(mrow, INT32_MIN);
         hipLaunchKernelGGL(k_scan_window, dim3(grid_for(wn)), dim3(256), 0, stream_, d, cols + begin, (int32_t)wn,
                            fl);
-        const int cg = grid_for(wn);
+        // Columns in the worklist, at most: a round's additions are losers and displaced pivots,
+        // one for each column that claimed, and only they can claim again.  The grids follow it:
+        // an empty workgroup is still placed with its LDS (k_add_long and k_add_huge with empty
+        // lists: 2.4 and 3.0 us with a small grid, 4.3 and 4.6 us with 512 and 256 workgroups).
+        int64_t bound = wn;
         int r = 0;
         for (;;) {
+          const int cg = grid_for(bound);
+          const int add_grid = (int)std::min<int64_t>(add_grid_max, (bound + wpg - 1) / wpg);
+          const int long_grid = (int)std::min<int64_t>(long_grid_max, bound);
+          const int huge_grid = (int)std::min<int64_t>(kHugeGroups, bound);
           for (int t = 0; t < rounds_per_sync; t++, r++) {
-            hipLaunchKernelGGL(k_claim, dim3(cg), dim3(256), 0, stream_, d, r);
-            hipLaunchKernelGGL(k_pivmeta, dim3(cg), dim3(256), 0, stream_, d, r);
+            if (bound <= kOneClaim) {
+              hipLaunchKernelGGL(k_claim_publish, dim3(1), dim3(1024), 0, stream_, d, r);
+            } else {
+              hipLaunchKernelGGL(k_claim, dim3(cg), dim3(256), 0, stream_, d, r);
+              hipLaunchKernelGGL(k_pivmeta, dim3(cg), dim3(256), 0, stream_, d, r);
+            }
             if (timing_) HIPCHK(hipEventRecord(ev_[4 * t], stream_));
             if (wpg == 2)
               hipLaunchKernelGGL(k_add<2>, dim3(add_grid), dim3(kWave * 2), 0, stream_, d, r, fl);
@@ -3068,7 +3095,7 @@ int Engine::page_loop(Dev& d, const ssq_params& p, int32_t maxdim, const LoopPla
             if (timing_) HIPCHK(hipEventRecord(ev_[4 * t + 1], stream_));
             hipLaunchKernelGGL(k_add_long, dim3(long_grid), dim3(kLongThreads), 0, stream_, d, r, fl);
             if (timing_) HIPCHK(hipEventRecord(ev_[4 * t + 2], stream_));
-            hipLaunchKernelGGL(k_add_huge, dim3(kHugeGroups), dim3(kLongThreads), 0, stream_, d, r, fl);
+            hipLaunchKernelGGL(k_add_huge, dim3(huge_grid), dim3(kLongThreads), 0, stream_, d, r, fl);
             if (timing_) HIPCHK(hipEventRecord(ev_[4 * t + 3], stream_));
           }
           HIPCHK(hipGetLastError());
@@ -3099,7 +3126,8 @@ int Engine::page_loop(Dev& d, const ssq_params& p, int32_t maxdim, const LoopPla
             oom = true;
             break;
           }
-          if (host_ctr_[cw::kW + (r & 1)] == 0) break;
+          bound = host_ctr_[cw::kW + (r & 1)];
+          if (bound == 0) break;
           if (r > (1 << 24)) {
             err_ = "page did not converge";
             return SSQ_EDEVICE;
