@@ -1021,6 +1021,9 @@ int ripsco_count(RipsCo* B, hipStream_t s, int count, const float* d_pts, const 
 // Cells of one group: a bound well inside the engine's int32 cell ids, and small enough that
 // the per-row tables of two consecutive groups' sizes fit beside each other as buffers grow.
 constexpr int64_t kGroupCells = (int64_t)1 << 30;
+// groups of a call that kGroupCells would leave on fewer groups than streams (ripsco_reduce)
+constexpr int64_t kSplitCells = (int64_t)1 << 23;
+constexpr int kSplitGroups = 6, kSplitStreams = 3;
 // device bytes each engine keeps for its huge-column bit sets (k_add_huge regions)
 constexpr int64_t kHugeRegionBytes = (int64_t)256 << 24;
 
@@ -1424,35 +1427,54 @@ int ripsco_reduce(RipsCo* const* Bs, PrebuiltTarget* const* engs, int nstreams, 
                                           std::max(nstreams, B->budget_streams));
   }
   // Groups: clouds by decreasing triangle count, consecutive ones while the group's estimated
-  // bytes fit the budget and its cells stay below kGroupCells.  The largest clouds (whose
-  // reductions hold the longest chains of additions) share groups, and the groups run on the
-  // streams side by side.
+  // bytes fit the budget and its cells stay below a limit.  The groups run on the streams side
+  // by side.  A group's rounds each last as long as the longest chase in them, which one
+  // workgroup runs, and clouds that share a group add up those times: 40 clouds of 64-2048
+  // points took 110 ms in one group, their longest alone 55 ms.  So where kGroupCells leaves
+  // streams without a group, the clouds are split further, into about kSplitGroups groups of
+  // at least kSplitCells cells (a group's launches and synchronisations are about 1 ms, the work
+  // on 8 million cells 2 ms or more).  Split calls take kSplitStreams streams: a process with
+  // streams of its own has more than its four hardware queues, and a short group then waits
+  // behind another's long chase (the call above: one group 130 ms, 3 streams 87-98, 4 107-120).
   std::vector<int> order((size_t)count);
   for (int c = 0; c < count; c++) order[(size_t)c] = c;
   std::stable_sort(order.begin(), order.end(),
                    [&](int x, int y) { return B->h_tris[(size_t)x] > B->h_tris[(size_t)y]; });
   std::vector<std::pair<int, int>> groups;  // [begin, end) in order
-  for (int i0 = 0; i0 < count;) {
-    int i1 = i0;
-    int64_t nv = 0, ne = 0, nt = 0, n2 = 0, ew = 0;
-    while (i1 < count) {
-      const int c = order[(size_t)i1];
-      const int64_t n = pbase[c + 1] - pbase[c], E = B->h_edges[(size_t)c], T = B->h_tris[(size_t)c];
-      const int64_t W = (n + 63) / 64;
-      const double bytes = group_bytes(nv + n, ne + E, nt + T, n2 + n * n, ew + E * W, (nt + T) / 16);
-      const bool fits = nv + n + ne + E + nt + T <= kGroupCells && bytes <= (double)mem_budget;
-      if (!fits && i1 > i0) break;
-      nv += n;
-      ne += E;
-      nt += T;
-      n2 += n * n;
-      ew += E * W;
-      i1++;
-      if (!fits) break;  // one cloud alone: try it anyway
+  auto make_groups = [&](int64_t cells) {
+    groups.clear();
+    for (int i0 = 0; i0 < count;) {
+      int i1 = i0;
+      int64_t nv = 0, ne = 0, nt = 0, n2 = 0, ew = 0;
+      while (i1 < count) {
+        const int c = order[(size_t)i1];
+        const int64_t n = pbase[c + 1] - pbase[c], E = B->h_edges[(size_t)c], T = B->h_tris[(size_t)c];
+        const int64_t W = (n + 63) / 64;
+        const double bytes = group_bytes(nv + n, ne + E, nt + T, n2 + n * n, ew + E * W, (nt + T) / 16);
+        const bool fits = nv + n + ne + E + nt + T <= cells && bytes <= (double)mem_budget;
+        if (!fits && i1 > i0) break;
+        nv += n;
+        ne += E;
+        nt += T;
+        n2 += n * n;
+        ew += E * W;
+        i1++;
+        if (!fits) break;  // one cloud alone: try it anyway
+      }
+      groups.emplace_back(i0, i1);
+      i0 = i1;
     }
-    groups.emplace_back(i0, i1);
-    i0 = i1;
+  };
+  make_groups(kGroupCells);
+  int workers = nstreams;
+  if ((int)groups.size() < nstreams) {
+    int64_t cells = 0;
+    for (int c = 0; c < count; c++)
+      cells += pbase[c + 1] - pbase[c] + B->h_edges[(size_t)c] + B->h_tris[(size_t)c];
+    make_groups(std::min(kGroupCells, std::max(kSplitCells, cells / kSplitGroups)));
+    workers = std::min(nstreams, kSplitStreams);
   }
+  workers = std::min(workers, (int)groups.size());
   std::vector<int64_t> counts((size_t)count, 0);
   std::vector<ssq_stats> accs((size_t)nstreams);
   std::vector<std::string> errs((size_t)nstreams);
@@ -1486,7 +1508,7 @@ int ripsco_reduce(RipsCo* const* Bs, PrebuiltTarget* const* engs, int nstreams, 
     }
   };
   std::vector<std::thread> pool;
-  for (int k = 1; k < nstreams; k++) pool.emplace_back(worker, k);
+  for (int k = 1; k < workers; k++) pool.emplace_back(worker, k);
   worker(0);
   for (auto& t : pool) t.join();
   for (int k = 0; k < nstreams; k++)

@@ -35,3 +35,22 @@ def test_claim_rounds(block, dualize):
     got = h.reduce(S.Matrix(m.colptr, m.rows, m.dims), S.params(dualize=dualize, ss_block_size=block))[0]
     h.close()
     assert np.array_equal(got, O.twist_pairs(m))
+
+
+@pytest.mark.parametrize("sizes", [(900, 60), (900, 850, 64, 800, 3)])
+def test_call_split_over_streams(monkeypatch, sizes):
+    """A call of more than 8 million cells is split into groups on several streams: pairs as on one
+    stream, where it is one group."""
+    rng = np.random.default_rng(len(sizes))
+    clouds = [(rng.random((n, 3)).astype(np.float32), 0.55) for n in sizes]
+    results = []
+    for streams in ("1", "4"):
+        monkeypatch.setenv("SSQ_RIPS_STREAMS", streams)
+        h = S.Handle(0)
+        *out, st = h.batch_reduce_points(clouds, 2, S.params(dualize=1), stats=True)
+        h.close()
+        results.append((out[0] if len(out) == 1 else out, st["n_pages"]))
+    (one, g1), (many, g4) = results
+    assert g1 == 1 and g4 > 1
+    for (a, ae), (b, be) in zip(one, many):
+        assert np.array_equal(a, b) and np.array_equal(ae, be)
