@@ -1812,8 +1812,7 @@ __global__ void k_run_len(int64_t n, int64_t nnz, const uint32_t* keys, const in
 __device__ void heapsort_i32(int32_t* a, int64_t n);
 
 // Sort every segment v[off[s] : off[s+1]) ascending.  Segments longer than a lane's share
-// are sorted by a wavefront: bitonic in registers up to 64 entries, in LDS up to kSortLds,
-// heapsort by one lane beyond (rare).
+// are sorted by a wavefront.
 constexpr int kSortLds = 2048;
 __device__ void heapsort_i32(int32_t* a, int64_t n) {
   auto sift = [&](int64_t i, int64_t m) {
@@ -1834,6 +1833,46 @@ __device__ void heapsort_i32(int32_t* a, int64_t n) {
     a[0] = a[m];
     a[m] = t;
     sift(0, m);
+  }
+}
+
+// One wavefront sorts v[0, len) ascending: bitonic in registers up to 64 entries, in buf
+// (kSortLds entries of LDS) up to kSortLds, heapsort by one lane beyond (rare).
+__device__ void wave_sort_list(int32_t* v, int64_t len, int32_t* buf) {
+  const int lane = lane_id();
+  if (len <= kWave) {
+    int32_t x = lane < len ? v[lane] : 0x7fffffff;
+    for (int k = 2; k <= kWave; k <<= 1)
+      for (int j = k >> 1; j > 0; j >>= 1) {
+        const int32_t y = __shfl_xor(x, j, kWave);
+        const bool up = (lane & k) == 0, lower = (lane & j) == 0;
+        x = (lower == up) ? min(x, y) : max(x, y);
+      }
+    if (lane < len) v[lane] = x;
+  } else if (len <= kSortLds) {
+    int P = kWave;
+    while (P < len) P <<= 1;
+    for (int i = lane; i < P; i += kWave) buf[i] = i < len ? v[i] : 0x7fffffff;
+    wave_sync();
+    for (int k = 2; k <= P; k <<= 1)
+      for (int j = k >> 1; j > 0; j >>= 1) {
+        for (int i = lane; i < P; i += kWave) {
+          const int l = i ^ j;
+          if (l > i) {
+            const int32_t a = buf[i], c = buf[l];
+            const bool asc = (i & k) == 0;
+            if ((a > c) == asc) {
+              buf[i] = c;
+              buf[l] = a;
+            }
+          }
+        }
+        wave_sync();
+      }
+    for (int i = lane; i < len; i += kWave) v[i] = buf[i];
+    wave_sync();
+  } else if (lane == 0) {
+    heapsort_i32(v, len);
   }
 }
 
@@ -1871,40 +1910,7 @@ __global__ void __launch_bounds__(256) k_sort_segments(int64_t nseg, const int64
       const int64_t s = g0 + src;
       const int64_t b = off[s];
       const int64_t len = off[s + 1] - b;
-      if (len <= kWave) {
-        int32_t x = lane < len ? v[b + lane] : 0x7fffffff;
-        for (int k = 2; k <= kWave; k <<= 1)
-          for (int j = k >> 1; j > 0; j >>= 1) {
-            const int32_t y = __shfl_xor(x, j, kWave);
-            const bool up = (lane & k) == 0, lower = (lane & j) == 0;
-            x = (lower == up) ? min(x, y) : max(x, y);
-          }
-        if (lane < len) v[b + lane] = x;
-      } else if (len <= kSortLds) {
-        int P = kWave;
-        while (P < len) P <<= 1;
-        for (int i = lane; i < P; i += kWave) buf[i] = i < len ? v[b + i] : 0x7fffffff;
-        wave_sync();
-        for (int k = 2; k <= P; k <<= 1)
-          for (int j = k >> 1; j > 0; j >>= 1) {
-            for (int i = lane; i < P; i += kWave) {
-              const int l = i ^ j;
-              if (l > i) {
-                const int32_t a = buf[i], c = buf[l];
-                const bool asc = (i & k) == 0;
-                if ((a > c) == asc) {
-                  buf[i] = c;
-                  buf[l] = a;
-                }
-              }
-            }
-            wave_sync();
-          }
-        for (int i = lane; i < len; i += kWave) v[b + i] = buf[i];
-        wave_sync();
-      } else if (lane == 0) {
-        heapsort_i32(v + b, len);
-      }
+      wave_sort_list(v + b, len, buf);
     }
   }
 }
@@ -2237,12 +2243,23 @@ __device__ __forceinline__ int32_t hash_find(const Key128* keys, const int32_t* 
 // (dim+1)-simplex whose other facets are all cells with index < s (kernel.h:203-292;
 // Lemma: the youngest facet of a boundary cycle is positive).  Neighbours of the vertex
 // with the fewest neighbours are walked from the highest id down, at most max_iter of them.
-__global__ void k_hd_clear(int64_t n, int32_t dim, const int32_t* dims, const uint8_t* removed,
-                           const int32_t* vs, int bits, const int64_t* adj_off, const int32_t* adj,
-                           const Key128* keys, const int32_t* vals, uint64_t mask, int32_t max_iter,
-                           uint8_t* hdclear, uint32_t* ncleared) {
-  GRID_STRIDE(c, n) {
-    if (dims[c] != dim || removed[c]) continue;
+// A neighbour costs chains of dependent loads (binary searches, hash probes), so kHdLanes lanes
+// take a cell's neighbours side by side; the order does not matter, one that serves is enough.
+// cells lists the max-dim cells (217,000 tetrahedra: 266 us by a lane each, now 197 us).
+constexpr int kHdLanes = 8;
+__global__ void __launch_bounds__(256) k_hd_clear(int64_t ncells, const int32_t* cells, int32_t dim,
+                                                  const uint8_t* removed, const int32_t* vs, int bits,
+                                                  const int64_t* adj_off, const int32_t* adj, const Key128* keys,
+                                                  const int32_t* vals, uint64_t mask, int32_t max_iter,
+                                                  uint8_t* hdclear, uint32_t* ncleared) {
+  __shared__ uint32_t found;
+  if (threadIdx.x == 0) found = 0u;
+  __syncthreads();
+  const int sub = threadIdx.x % kHdLanes, shift = lane_id() & ~(kHdLanes - 1);
+  for (int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kHdLanes; i < ncells;
+       i += (int64_t)gridDim.x * blockDim.x / kHdLanes) {
+    const int64_t c = cells[i];
+    if (removed[c]) continue;
     const int32_t* v = vs + c * kMaxVerts;
     if (v[0] < 0) continue;
     const int nv = dim + 1;
@@ -2250,11 +2267,12 @@ __global__ void k_hd_clear(int64_t n, int32_t dim, const int32_t* dims, const ui
     for (int t = 1; t < nv; t++)
       if (adj_off[v[t] + 1] - adj_off[v[t]] < adj_off[v[best] + 1] - adj_off[v[best]]) best = t;
     const int64_t b0 = adj_off[v[best]];
-    int64_t p = adj_off[v[best] + 1] - 1;
+    const int64_t tries = min((int64_t)max_iter, adj_off[v[best] + 1] - b0);
     bool cleared = false;
-    for (int32_t it = 0; it < max_iter && p >= b0 && !cleared; it++, p--) {
-      const int32_t x = adj[p];
-      bool ok = true;
+    for (int64_t it = 0; it < tries && !cleared; it += kHdLanes) {  // alike in the cell's lanes
+      bool all = it + sub < tries;
+      const int32_t x = all ? adj[adj_off[v[best] + 1] - 1 - it - sub] : -1;
+      bool ok = all;
       for (int t = 0; t < nv && ok; t++) {
         if (t == best) continue;
         if (v[t] == x) { ok = false; break; }
@@ -2267,7 +2285,6 @@ __global__ void k_hd_clear(int64_t n, int32_t dim, const int32_t* dims, const ui
         }
         ok = lo < adj_off[v[t] + 1] && adj[lo] == x;
       }
-      if (!ok) continue;
       // tau = v + {x}; every facet other than s itself must exist with index < c
       int32_t tau[kMaxVerts + 1];
       int k = 0;
@@ -2280,7 +2297,7 @@ __global__ void k_hd_clear(int64_t n, int32_t dim, const int32_t* dims, const ui
         tau[k++] = v[t];
       }
       if (!put) tau[k++] = x;
-      bool all = true;
+      all = ok;
       for (int drop = 0; drop <= nv && all; drop++) {
         if (tau[drop] == x) continue;  // that facet is s itself
         int32_t f[kMaxVerts];
@@ -2290,13 +2307,15 @@ __global__ void k_hd_clear(int64_t n, int32_t dim, const int32_t* dims, const ui
         const int32_t col = hash_find(keys, vals, mask, pack_key(f, nv, bits));
         all = col >= 0 && col < c;
       }
-      if (all) cleared = true;
+      cleared = ((__ballot(all) >> shift) & ((1u << kHdLanes) - 1)) != 0;
     }
-    if (cleared) {
+    if (cleared && sub == 0) {
       hdclear[c] = 1;
-      atomicAdd(ncleared, 1u);
+      atomicAdd(&found, 1u);
     }
   }
+  __syncthreads();
+  if (threadIdx.x == 0 && found) atomicAdd(ncleared, found);
 }
 
 // adjacency (CSR over vertex ranks) of the edges still in the complex
@@ -2317,19 +2336,13 @@ __global__ void k_adj_fill(int64_t ne, const int32_t* eu, const int32_t* ev, con
     adj[off[b] + (int64_t)atomicAdd(&fill[b], 1ull)] = a;
   }
 }
-__global__ void k_adj_sort(int64_t nv, const int64_t* off, int32_t* adj) {
-  GRID_STRIDE(a, nv) {
-    const int64_t b = off[a], e = off[a + 1];
-    for (int64_t i = b + 1; i < e; i++) {
-      const int32_t x = adj[i];
-      int64_t j = i - 1;
-      while (j >= b && adj[j] > x) {
-        adj[j + 1] = adj[j];
-        j--;
-      }
-      adj[j + 1] = x;
-    }
-  }
+// Neighbour lists ascending, a wavefront each: a list holds up to the vertex count, so a lane's
+// insertion sort is quadratic in loads of its own (300 vertices at mean degree 40: 446 us, now 11 us).
+__global__ void __launch_bounds__(256) k_adj_sort(int64_t nv, const int64_t* off, int32_t* adj) {
+  __shared__ int32_t lds[4][kSortLds];
+  const int w = threadIdx.x / kWave;
+  for (int64_t a = (int64_t)blockIdx.x * 4 + w; a < nv; a += (int64_t)gridDim.x * 4)
+    wave_sort_list(adj + off[a], off[a + 1] - off[a], lds[w]);
 }
 __global__ void k_vrank_ends(int64_t ne, const int32_t* vrank, int32_t* eu, int32_t* ev, uint32_t* bad) {
   GRID_STRIDE(i, ne) {
@@ -2841,12 +2854,12 @@ int Engine::guided_clear(Dev& d, int64_t n, int32_t maxdim, const int32_t* d_dim
   HIPCHK(hipMemcpyAsync(aoff, deg.data(), sizeof(int64_t) * (nv + 1), hipMemcpyHostToDevice, stream_));
   hipLaunchKernelGGL(k_adj_fill, dim3(grid_for(std::max<int64_t>(ne, 1))), dim3(256), 0, stream_, ne, eu, ev, ecols,
                      d.removed, aoff, fill, adj);
-  hipLaunchKernelGGL(k_adj_sort, dim3(grid_for(nv)), dim3(256), 0, stream_, nv, aoff, adj);
+  hipLaunchKernelGGL(k_adj_sort, dim3(grid_for(std::max<int64_t>(nv, 1) * kWave)), dim3(256), 0, stream_, nv, aoff, adj);
   // hash of max-dim cells
   int64_t nmax = 0;
   {
     int64_t cnt[1];
-    rc = compact(n, 1, KeyDimEq{d_dims, maxdim}, EmitIndex{ecols}, cnt);  // ecols reused as scratch
+    rc = compact(n, 1, KeyDimEq{d_dims, maxdim}, EmitIndex{ecols}, cnt);  // the edges' list is done with
     if (rc) return rc;
     nmax = cnt[0];
   }
@@ -2860,8 +2873,8 @@ int Engine::guided_clear(Dev& d, int64_t n, int32_t maxdim, const int32_t* d_dim
   hipLaunchKernelGGL(k_hash_insert, dim3(grid_for(n)), dim3(256), 0, stream_, n, maxdim, d_dims, d.removed, vs, bits,
                      keys, vals, (uint64_t)(hsize - 1));
   DCHK(dfill(d.ctr + cw::kHdCleared, 0, sizeof(uint32_t)));
-  hipLaunchKernelGGL(k_hd_clear, dim3(grid_for(n)), dim3(256), 0, stream_, n, maxdim, d_dims, d.removed, vs, bits,
-                     aoff, adj, keys, vals, (uint64_t)(hsize - 1), p.max_iteration, hd, d.ctr + cw::kHdCleared);
+  hipLaunchKernelGGL(k_hd_clear, dim3(grid_for(std::max<int64_t>(nmax, 1) * kHdLanes)), dim3(256), 0, stream_, nmax,
+                     ecols, maxdim, d.removed, vs, bits, aoff, adj, keys, vals, (uint64_t)(hsize - 1), p.max_iteration, hd, d.ctr + cw::kHdCleared);
   HIPCHK(hipGetLastError());
   rc = sync_read(d.ctr + cw::kHdCleared, 1);
   if (rc) return rc;
