@@ -663,6 +663,12 @@ struct Running {
   __device__ __forceinline__ uint64_t lost() const {
     return alive ? held & ~alive & ~((alive & -alive) - 1) : 0ull;
   }
+  // Lanes of the window's rows that left the column below its low.  While the low is an overlay row,
+  // a pivot may bring back a window row that left at the top, and all of these are lost at once: it is
+  // their number, not that of the lost ones, that a pivot of b rows raises by no more than b (together
+  // with the overlay's rows), and that only falls as the low does.  A flush is rare either way: at most
+  // 470 in 24 sparse clouds of 64-4096 points, 5 of them for this count's sake.
+  __device__ __forceinline__ uint64_t left(int32_t low) const { return held & ~alive & __ballot(top_row < low); }
   // Row x (the same in every lane) into the column or out of it.
   __device__ __forceinline__ void toggle(int32_t x) {
     const uint64_t in_window = __ballot(top_row == x);
@@ -830,8 +836,8 @@ __global__ void __launch_bounds__(kWave * kAddWaves) k_add(Dev d, int r, int32_t
           open_window();
         }
         if (b_len <= kTinyRows) {
-          // a flush puts the window's lost rows (64 at most) and the overlay's into one overlay
-          if (__popcll(q.used) + __popcll(q.lost()) + b_len > kWave) {
+          // a flush puts the window's lost rows and the overlay's into one overlay of 64 lanes
+          if (__popcll(q.used) + __popcll(q.left(l)) + b_len > kWave) {
             flush();
             open_window();
           }
