@@ -47,6 +47,7 @@
 #include <thread>
 #include <vector>
 
+#include "ssq_groups.h"
 #include "ssq_internal.h"
 #include "ssq_kernels.h"
 #include "ssq_sort.h"
@@ -1018,30 +1019,6 @@ int ripsco_count(RipsCo* B, hipStream_t s, int count, const float* d_pts, const 
   return SSQ_OK;
 }
 
-// Cells of one group: a bound well inside the engine's int32 cell ids, and small enough that
-// the per-row tables of two consecutive groups' sizes fit beside each other as buffers grow.
-constexpr int64_t kGroupCells = (int64_t)1 << 30;
-// groups of a call that kGroupCells would leave on fewer groups than streams (ripsco_reduce)
-constexpr int64_t kSplitCells = (int64_t)1 << 23;
-constexpr int kSplitGroups = 6, kSplitStreams = 3;
-// device bytes each engine keeps for its huge-column bit sets (k_add_huge regions)
-constexpr int64_t kHugeRegionBytes = (int64_t)256 << 24;
-
-// Device bytes of one group, by the buffers below (the engine's included), with the slack of
-// their geometric growth (1.5x for the engine's buffers, 1.25x for the builder's).
-static double group_bytes(int64_t nv, int64_t ne, int64_t nt, int64_t n2, int64_t ew, int64_t tie_guess) {
-  const double rows = 2.0 * ne + 3.0 * nt;
-  const double engine = 4.0 * rows * 2.0                // pool: rows, then the arena (holds the staging)
-                        + 42.0 * (double)(nv + ne + nt) // per-row tables: piv, leftone, flags, pivmeta
-                        + 40.0 * (double)(nv + ne);     // per-column state and lists
-  const double builder = 4.0 * (double)nt               // tie remap
-                         + 4.0 * (double)n2             // rank matrices
-                         + 10.0 * (double)ew            // Q bitsets and prefix counts
-                         + 120.0 * (double)ne + 80.0 * (double)nv  // edge keys, runs, lists, lengths
-                         + 32.0 * (double)tie_guess;
-  return 1.5 * engine + 1.25 * builder + 64.0 * 1048576.0;
-}
-
 // One group: clouds[0 .. G) (indices into the sizing pass S), built and reduced on stream s;
 // each cloud's pairs go to stage at its slot, their count to counts[cloud].
 static int rc_group(RipsCo* B, const RipsCo* S, PrebuiltTarget* eng, hipStream_t s, const int* clouds, int G,
@@ -1426,55 +1403,13 @@ int ripsco_reduce(RipsCo* const* Bs, PrebuiltTarget* const* engs, int nstreams, 
     mem_budget = std::max<int64_t>(1, (B->budget - (int64_t)extra * kHugeRegionBytes) /
                                           std::max(nstreams, B->budget_streams));
   }
-  // Groups: clouds by decreasing triangle count, consecutive ones while the group's estimated
-  // bytes fit the budget and its cells stay below a limit.  The groups run on the streams side
-  // by side.  A group's rounds each last as long as the longest chase in them, which one
-  // workgroup runs, and clouds that share a group add up those times: 40 clouds of 64-2048
-  // points took 110 ms in one group, their longest alone 55 ms.  So where kGroupCells leaves
-  // streams without a group, the clouds are split further, into about kSplitGroups groups of
-  // at least kSplitCells cells (a group's launches and synchronisations are about 1 ms, the work
-  // on 8 million cells 2 ms or more).  Split calls take kSplitStreams streams: a process with
-  // streams of its own has more than its four hardware queues, and a short group then waits
-  // behind another's long chase (the call above: one group 130 ms, 3 streams 87-98, 4 107-120).
-  std::vector<int> order((size_t)count);
-  for (int c = 0; c < count; c++) order[(size_t)c] = c;
-  std::stable_sort(order.begin(), order.end(),
-                   [&](int x, int y) { return B->h_tris[(size_t)x] > B->h_tris[(size_t)y]; });
-  std::vector<std::pair<int, int>> groups;  // [begin, end) in order
-  auto make_groups = [&](int64_t cells) {
-    groups.clear();
-    for (int i0 = 0; i0 < count;) {
-      int i1 = i0;
-      int64_t nv = 0, ne = 0, nt = 0, n2 = 0, ew = 0;
-      while (i1 < count) {
-        const int c = order[(size_t)i1];
-        const int64_t n = pbase[c + 1] - pbase[c], E = B->h_edges[(size_t)c], T = B->h_tris[(size_t)c];
-        const int64_t W = (n + 63) / 64;
-        const double bytes = group_bytes(nv + n, ne + E, nt + T, n2 + n * n, ew + E * W, (nt + T) / 16);
-        const bool fits = nv + n + ne + E + nt + T <= cells && bytes <= (double)mem_budget;
-        if (!fits && i1 > i0) break;
-        nv += n;
-        ne += E;
-        nt += T;
-        n2 += n * n;
-        ew += E * W;
-        i1++;
-        if (!fits) break;  // one cloud alone: try it anyway
-      }
-      groups.emplace_back(i0, i1);
-      i0 = i1;
-    }
-  };
-  make_groups(kGroupCells);
-  int workers = nstreams;
-  if ((int)groups.size() < nstreams) {
-    int64_t cells = 0;
-    for (int c = 0; c < count; c++)
-      cells += pbase[c + 1] - pbase[c] + B->h_edges[(size_t)c] + B->h_tris[(size_t)c];
-    make_groups(std::min(kGroupCells, std::max(kSplitCells, cells / kSplitGroups)));
-    workers = std::min(nstreams, kSplitStreams);
-  }
-  workers = std::min(workers, (int)groups.size());
+  std::vector<CloudSize> sizes((size_t)count);
+  for (int c = 0; c < count; c++)
+    sizes[(size_t)c] = {pbase[c + 1] - pbase[c], B->h_edges[(size_t)c], B->h_tris[(size_t)c]};
+  const GroupPlan plan = plan_groups(sizes, mem_budget, nstreams);
+  const std::vector<int>& order = plan.order;
+  const std::vector<std::pair<int, int>>& groups = plan.groups;
+  const int workers = plan.workers;
   std::vector<int64_t> counts((size_t)count, 0);
   std::vector<ssq_stats> accs((size_t)nstreams);
   std::vector<std::string> errs((size_t)nstreams);
