@@ -79,8 +79,10 @@ typedef struct ssq_stats {
   int64_t n_pages;       /* pages run                                                  */
   int64_t n_rounds;      /* claim/add rounds run                                       */
   int64_t n_additions;   /* column additions performed                                 */
-  double add_bytes;      /* algorithmic bytes of the short additions (LDS merges):
-                            4(|a|+|b|+|a^b|)+24 each                                   */
+  double add_bytes;      /* algorithmic bytes of the short additions (by a wavefront, on chip):
+                            4(|a|+|b|+|a^b|)+24 each.  A column is counted as it is held: a row
+                            that two parts of it hold, and that is gone, counts in both until
+                            they meet, so the sum may exceed that of the sets           */
   int64_t store_bytes;   /* device bytes reserved for the column store                 */
   double t_add_kernel_ms; /* summed duration of the column-addition kernel launches, from
                              HIP events on the engine stream (SSQ_KERNEL_TIMING=1), else 0 */
@@ -91,7 +93,7 @@ typedef struct ssq_stats {
                              running column stays in the LDS bit set)                     */
   double t_add_long_kernel_ms; /* summed duration of the long-column kernel launches     */
   int64_t max_chain;      /* most additions one column made in one round                */
-  int64_t max_addition_len; /* largest |a|+|b| of one addition                          */
+  int64_t max_addition_len; /* largest |a|+|b| of one addition (|b| alone where a is a bit set) */
   int64_t n_huge_additions; /* additions of columns whose rows spread past the LDS window
                                (an LDS window over a device-memory bit set)                */
   double huge_bytes;      /* bytes those additions move: 4|b|+24 each (the pivot's rows; the

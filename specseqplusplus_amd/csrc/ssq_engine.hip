@@ -733,7 +733,9 @@ __global__ void __launch_bounds__(kWave * kAddWaves) k_add(Dev d, int r, int32_t
     bool failed = false;
     int32_t* sA = bufA;
     int32_t* sO = bufO;
-    uint32_t chain = 0, moved = 0;
+    uint32_t chain = 0;
+    uint64_t moved = 0;    // entries read and written: a chase of millions of additions passes 32 bits
+    int32_t rows = a_len;  // the column's rows (not fewer): the base below its window, the window's, the overlay's
     bool deferred = false;
     Running q;
     int32_t top_at = -1;  // base index of the window's lane 0
@@ -826,9 +828,7 @@ __global__ void __launch_bounds__(kWave * kAddWaves) k_add(Dev d, int r, int32_t
       // merges with a load in flight waits for it
       spec_p = d.piv[max(cand, 0)];
       spec_pm = d.pivmeta[max(cand, 0)];
-      // the column's rows (not fewer): the base without its window, the window's, the overlay's
-      const int32_t before = in_lds ? max(top_at + 1 - kWave, 0) + __popcll(q.alive) + __popcll(q.used) : a_len;
-      if (before + b_len <= d.short_max) {
+      if (rows + b_len <= d.short_max) {
         if (!in_lds) {
           wave_copy(sA, d.pool + a_off, a_len);
           in_lds = true;
@@ -909,8 +909,10 @@ __global__ void __launch_bounds__(kWave * kAddWaves) k_add(Dev d, int r, int32_t
       const int32_t base2 = next ? __builtin_amdgcn_readlane(q.top_row, __ffsll((unsigned long long)next) - 1) : -1;
       a2 = l_base ? max(base2, top_o) : base2;
       chain += 1;
-      max_len = max(max_len, (uint32_t)(before + b_len));
-      moved += (uint32_t)(2 * before + b_len);
+      max_len = max(max_len, (uint32_t)(rows + b_len));
+      moved += (uint32_t)(rows + b_len);
+      rows = max(top_at + 1 - kWave, 0) + __popcll(q.alive) + __popcll(q.used);
+      moved += (uint32_t)rows;
       if (l < 0 || l < minrow) break;
     }
     max_chain = max(max_chain, chain);

@@ -202,3 +202,36 @@ def test_returning_rows(h, name):
     mm = S.Matrix(m.colptr, m.rows, m.dims)
     for kw in ({"dualize": 0, "model": 0}, {"dualize": 1, "model": 0}, {"dualize": 0, "model": 0, "queue_size": 1}):
         assert np.array_equal(h.reduce(mm, S.params(**kw))[0], ref), kw
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["review", "steps", "len63_rows16", "len64_rows2", "len200_rows15"])
+def test_bytes_of_a_chase(h, name):
+    """add_bytes is 4(|a| + |b| + |a ^ b|) + 24 for each addition of the one chase (no row of these
+    columns is in the overlay and in the base at once)."""
+    column, pivots = CASES[name]
+    cols = [sorted(p) for p in pivots] + [sorted(column)]
+    m = O.Matrix.from_columns([[] for _ in range(1001)] + cols, [0] * 1001 + [1] * len(cols))
+    st = h.reduce(S.Matrix(m.colptr, m.rows, m.dims), S.params(model=0, ss_block_size=1 << 30), stats=True)[-1]
+    by_low, a, want, longest = {max(p): p for p in pivots}, set(column), 0, 0
+    while a and max(a) in by_low:
+        b = by_low[max(a)]
+        want += 4 * (len(a) + len(b) + len(a ^ b)) + 24
+        longest = max(longest, len(a) + len(b))
+        a = a ^ b
+    assert (st["n_additions"], st["add_bytes"], st["max_addition_len"]) == (len(pivots), want, longest)
+
+
+@pytest.mark.gpu
+def test_bytes_of_a_long_chase(h):
+    """A chase whose entries pass 32 bits: 2.2 million pivots of two rows, a column of 1001."""
+    steps, kept = 2_200_000, 1000
+    n = kept + steps + 1
+    chain = np.stack([np.arange(kept, n - 1), np.arange(kept + 1, n)], 1)[::-1]  # {low - 1, low}
+    rows = np.concatenate([chain.ravel(), np.arange(kept), [n - 1]]).astype(np.int32)
+    colptr = np.concatenate([np.zeros(n, np.int64), 2 * np.arange(steps + 1), [len(rows)]]).astype(np.int64)
+    dims = np.concatenate([np.zeros(n), np.ones(steps + 1)]).astype(np.int32)
+    pairs, _, st = h.reduce(S.Matrix(colptr, rows, dims), S.params(model=0, ss_block_size=1 << 30), stats=True)
+    assert len(pairs) == steps + 1 and pairs[0].tolist() == [kept, n + steps]
+    a = kept + 1
+    assert (st["n_additions"], st["add_bytes"]) == (steps, steps * (4 * (2 * a + 2) + 24))
