@@ -54,6 +54,12 @@ struct Graph {
   std::vector<int64_t> toff;
   Tri* tri = nullptr;  // edge e's triangles: [toff[e], toff[e] + tcnt[e])
   std::vector<int32_t> tcnt;
+  // No loops and no two edges with the same ends.  Otherwise the tables have more than one answer
+  // for a pair of vertices (edge_id(x, w) need not be edge_id(w, x)), the third vertices are kept in tx,
+  // and candidates are tried one by one: such lists keep the edges that the merges of adjacency
+  // lists, or the bit sets, give for them.
+  bool simple = true;
+  std::vector<int32_t> tx;
   std::vector<int32_t> eu, ev, ex;  // ends, and their exclusive or
   // With at most kBitsetVertices vertices: each neighbourhood as a bit set, W words per vertex.
   // Each word has beside it where its first neighbour stands in nbr and eid, so that finding
@@ -99,6 +105,17 @@ int64_t common_e(const Graph& g, int32_t e, Valid valid, int32_t* out, int32_t* 
   const int32_t nt = g.tcnt[e], a = g.eu[e];
   // No branch on what is valid, which cannot be predicted: every entry is written, and k stands
   // still for those that are not (an edge has fewer triangles than the arrays have room).
+  if (!g.simple) {
+    const int32_t* tx = g.tx.data() + g.toff[e];
+    for (int32_t t = 0; t < nt; t++) {
+      const int32_t e1 = tri[t].ea, e2 = tri[t].eb;
+      if (!valid(e1) || !valid(e2)) continue;
+      ea[k] = e1;
+      eb[k] = e2;
+      out[k++] = tx[t];
+    }
+    return k;
+  }
   for (int32_t t = 0; t < nt; t++) {
     const int32_t e1 = tri[t].ea, e2 = tri[t].eb;
     ea[k] = e1;
@@ -185,6 +202,16 @@ bool dominated(const Graph& g, int32_t e, Valid valid, Work& wk, int32_t* witnes
   if (m <= 1) {
     if (m == 1) *witness = I[0];
     return m == 1;
+  }
+  if (!g.simple) {  // striking relies on an edge having one id from both its ends
+    const int32_t hint = *witness;
+    if (hint >= 0 && std::binary_search(I, I + m, hint) && uncovered(g, hint, I, m, valid) < 0) return true;
+    for (int64_t c = 0; c < m; c++) {
+      if (I[c] == hint || uncovered(g, I[c], I, m, valid) >= 0) continue;
+      *witness = I[c];
+      return true;
+    }
+    return false;
   }
   int64_t n = m;
   std::copy(I, I + m, C);
@@ -288,13 +315,20 @@ void collapse_edges(int64_t ne, const int32_t* u, const int32_t* v, uint8_t* kep
   };
   auto parallel_edges = [&](auto&& body) { parallel_range(ne, 1024, body); };
   // each vertex's neighbours ascending (they were filled in edge order)
+  std::atomic<bool> simple{true};
   parallel_range(nv, 16, [&](int64_t a) {
     thread_local std::vector<std::pair<int32_t, int32_t>> tmp;
     tmp.clear();
     for (int64_t p = g.off[a]; p < g.off[a + 1]; p++) tmp.emplace_back(g.nbr[p], g.eid[p]);
     std::sort(tmp.begin(), tmp.end());
-    for (int64_t p = g.off[a], k = 0; p < g.off[a + 1]; p++, k++) { g.nbr[p] = tmp[k].first; g.eid[p] = tmp[k].second; }
+    for (int64_t p = g.off[a], k = 0; p < g.off[a + 1]; p++, k++) {
+      g.nbr[p] = tmp[k].first;
+      g.eid[p] = tmp[k].second;
+      if (tmp[k].first == a || (k > 0 && tmp[k].first == tmp[k - 1].first))
+        simple.store(false, std::memory_order_relaxed);
+    }
   });
+  g.simple = simple;
   int64_t maxdeg = 1;
   for (int64_t a = 0; a < nv; a++) maxdeg = std::max(maxdeg, g.off[a + 1] - g.off[a]);
   g.eu = eu;
@@ -337,6 +371,7 @@ void collapse_edges(int64_t ne, const int32_t* u, const int32_t* v, uint8_t* kep
       thread_local TriBuffer keep;
       keep.reserve((size_t)cap[ne]);
       g.tri = keep.p;
+      if (!g.simple) g.tx.resize((size_t)cap[ne]);
       if (nv <= kBitsetVertices) {
         parallel_edges([&](int64_t e) {
           const int32_t a = eu[e], b = ev[e];
@@ -347,6 +382,7 @@ void collapse_edges(int64_t ne, const int32_t* u, const int32_t* v, uint8_t* kep
             while (m) {
               const int bit = __builtin_ctzll(m);
               const uint64_t below = (1ull << bit) - 1;
+              if (!g.simple) g.tx[(size_t)(tri - g.tri)] = (int32_t)(w * 64 + bit);
               *tri++ = Tri{g.eid[ra[w].pos + __builtin_popcountll(ra[w].bits & below)],
                            g.eid[rb[w].pos + __builtin_popcountll(rb[w].bits & below)]};
               m &= m - 1;
@@ -358,8 +394,8 @@ void collapse_edges(int64_t ne, const int32_t* u, const int32_t* v, uint8_t* kep
           thread_local std::vector<int32_t> ta, tb;
           ta.resize((size_t)maxdeg);
           tb.resize((size_t)maxdeg);
-          const int32_t k =
-              (int32_t)common(g, eu[e], ev[e], [](int32_t) { return true; }, (int32_t*)nullptr, ta.data(), tb.data());
+          int32_t* tx = g.simple ? nullptr : g.tx.data() + cap[e];
+          const int32_t k = (int32_t)common(g, eu[e], ev[e], [](int32_t) { return true; }, tx, ta.data(), tb.data());
           for (int32_t t = 0; t < k; t++) g.tri[cap[e] + t] = Tri{ta[t], tb[t]};
           g.tcnt[e] = k;
         });
@@ -418,6 +454,9 @@ void collapse_edges(int64_t ne, const int32_t* u, const int32_t* v, uint8_t* kep
   // the valid triangles of e, now critical, in wk: their other edges are tested again
   auto three_clique = [&](int32_t thresh, int32_t e, int32_t sid) {
     const uint8_t* crit = g.crit.data();
+    if (!g.simple)  // an edge may be in a triangle of its own: the test before did not see it as critical
+      wk.m = common_e(g, e, [thresh, crit](int32_t x) { return (x < thresh) | crit[x]; }, wk.I.data(), wk.ea.data(),
+                      wk.eb.data());
     const int32_t p = g.eu[e], q = g.ev[e];
     for (int64_t k = 0; k < wk.m; k++) {
       const int32_t e1 = wk.ea[k], e2 = wk.eb[k];  // e1 = (p, x) gains q, e2 = (q, x) gains p
