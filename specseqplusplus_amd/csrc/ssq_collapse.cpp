@@ -203,7 +203,10 @@ bool dominated(const Graph& g, int32_t e, Valid valid, Work& wk, int32_t* witnes
     if (m == 1) *witness = I[0];
     return m == 1;
   }
-  if (!g.simple) {  // striking relies on an edge having one id from both its ends
+  // Striking relies on an edge having one id from both its ends, and on the bit sets: without them an id
+  // is a binary search, and it pays to read one candidate's list after the other (17,000 vertices of
+  // mean degree 300: 5.6 s with the searches, 5.2 s this way, on 8 threads; in the plane 2.3 and 1.7 s).
+  if (!g.simple || !g.W) {
     const int32_t hint = *witness;
     if (hint >= 0 && std::binary_search(I, I + m, hint) && uncovered(g, hint, I, m, valid) < 0) return true;
     for (int64_t c = 0; c < m; c++) {
