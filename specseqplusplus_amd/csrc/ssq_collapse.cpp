@@ -38,6 +38,28 @@
 
 namespace {
 
+// Uninitialised storage in large pages where the system has them, grown as needed and never shrunk.
+template <typename T>
+struct Pages {
+  T* p = nullptr;
+  size_t cap = 0;
+  Pages() = default;
+  Pages(const Pages&) = delete;
+  Pages& operator=(const Pages&) = delete;
+  ~Pages() { std::free(p); }
+  void reserve(size_t n) {
+    if (n <= cap) return;
+    constexpr size_t kPage = size_t(1) << 21;
+    const size_t bytes = ((n + n / 4) * sizeof(T) + kPage - 1) / kPage * kPage;
+    std::free(p);
+    cap = 0;
+    p = (T*)std::aligned_alloc(kPage, bytes);
+    if (!p) throw std::bad_alloc();
+    madvise(p, bytes, MADV_HUGEPAGE);  // a hint: without it only slower
+    cap = bytes / sizeof(T);
+  }
+};
+
 struct Tri {
   int32_t ea, eb;
 };
@@ -68,29 +90,11 @@ struct Graph {
     uint64_t bits;
     int64_t pos;
   };
-  std::vector<Word> nb;
+  Pages<Word> nb;
   int64_t W = 0;
 };
-// Storage of the triangle lists, grown as needed and never shrunk, in large pages where the
-// system has them.
-struct TriBuffer {
-  Tri* p = nullptr;
-  size_t cap = 0;
-  ~TriBuffer() { std::free(p); }
-  void reserve(size_t n) {
-    if (n <= cap) return;
-    constexpr size_t kPage = size_t(1) << 21;
-    const size_t bytes = ((n + n / 4) * sizeof(Tri) + kPage - 1) / kPage * kPage;
-    std::free(p);
-    cap = 0;
-    p = (Tri*)std::aligned_alloc(kPage, bytes);
-    if (!p) throw std::bad_alloc();
-    madvise(p, bytes, MADV_HUGEPAGE);  // a hint: without it only slower
-    cap = bytes / sizeof(Tri);
-  }
-};
 constexpr int64_t kTriListMax = int64_t(1) << 28;  // entries (8 bytes each)
-constexpr int64_t kBitsetVertices = 16384;          // neighbourhood bit sets up to 32 MB
+constexpr int64_t kBitsetVertices = 16384;          // neighbourhood bit sets up to 64 MB
 
 template <typename Valid>
 int64_t common(const Graph& g, int32_t a, int32_t b, Valid valid, int32_t* out, int32_t* ea,
@@ -151,7 +155,7 @@ int64_t common(const Graph& g, int32_t a, int32_t b, Valid valid, int32_t* out, 
 // id of edge (u, v), or -1 (neighbours are ascending)
 inline int32_t edge_id(const Graph& g, int32_t u, int32_t v) {
   if (g.W) {
-    const Graph::Word& word = g.nb[(size_t)(u * g.W + (v >> 6))];
+    const Graph::Word& word = g.nb.p[u * g.W + (v >> 6)];
     const uint64_t bit = 1ull << (v & 63);
     if (!(word.bits & bit)) return -1;
     return g.eid[word.pos + __builtin_popcountll(word.bits & (bit - 1))];
@@ -342,15 +346,43 @@ void collapse_edges(int64_t ne, const int32_t* u, const int32_t* v, uint8_t* kep
     std::vector<int64_t> cap((size_t)ne + 1, 0);
     g.tcnt.assign((size_t)ne, 0);
     const int64_t W = (nv + 63) / 64;
-    std::vector<Graph::Word>& nb = g.nb;
+    // f(x, id of (a, x), id of (b, x)) for the common neighbours x of e = (a, b), ascending, by the bit
+    // sets: the set bits of one AND per word, or the shorter list's neighbours looked up in the other
+    // row where they are fewer than the words (16,000 vertices of mean degree 37: 340 ms in all on
+    // one thread by the words alone, 150 ms this way).
+    const auto each_common = [&](int64_t e, auto&& f) {
+      const int32_t a = eu[e], b = ev[e];
+      const Graph::Word *ra = g.nb.p + (int64_t)a * W, *rb = g.nb.p + (int64_t)b * W;
+      const auto id = [&](const Graph::Word& word, int bit) {
+        return g.eid[word.pos + __builtin_popcountll(word.bits & ((1ull << bit) - 1))];
+      };
+      const bool first = g.off[a + 1] - g.off[a] <= g.off[b + 1] - g.off[b];
+      const int32_t s = first ? a : b;
+      if (g.simple && g.off[s + 1] - g.off[s] < W) {
+        const Graph::Word* other = first ? rb : ra;
+        for (int64_t p = g.off[s]; p < g.off[s + 1]; p++) {
+          const int32_t x = g.nbr[p];
+          const Graph::Word& word = other[x >> 6];
+          if (!((word.bits >> (x & 63)) & 1)) continue;
+          const int32_t there = id(word, x & 63);
+          f(x, first ? g.eid[p] : there, first ? there : g.eid[p]);
+        }
+        return;
+      }
+      for (int64_t w = 0; w < W; w++)
+        for (uint64_t m = ra[w].bits & rb[w].bits; m; m &= m - 1) {
+          const int bit = __builtin_ctzll(m);
+          f(w * 64 + bit, id(ra[w], bit), id(rb[w], bit));
+        }
+    };
     if (nv <= kBitsetVertices) {
       g.W = W;
-      // neighbourhoods as bit sets: an edge's common neighbours are the set bits of one AND
-      // per word, in increasing order, and a neighbour's position in a sorted adjacency list
-      // is the popcount of the set bits below it (a prefix count per word plus one word)
-      nb.assign((size_t)(nv * W), Graph::Word{0, 0});
+      // neighbourhoods as bit sets: a neighbour's position in a sorted adjacency list is the
+      // popcount of the set bits below it (a prefix count per word plus one word)
+      g.nb.reserve((size_t)(nv * W));
       parallel_range(nv, 16, [&](int64_t a) {
-        Graph::Word* row = nb.data() + a * W;
+        Graph::Word* row = g.nb.p + a * W;
+        std::fill(row, row + W, Graph::Word{0, 0});
         for (int64_t p = g.off[a]; p < g.off[a + 1]; p++) row[g.nbr[p] >> 6].bits |= 1ull << (g.nbr[p] & 63);
         int64_t run = g.off[a];
         for (int64_t w = 0; w < W; w++) {
@@ -359,9 +391,8 @@ void collapse_edges(int64_t ne, const int32_t* u, const int32_t* v, uint8_t* kep
         }
       });
       parallel_edges([&](int64_t e) {  // exact counts first
-        const Graph::Word *ra = nb.data() + (int64_t)eu[e] * W, *rb = nb.data() + (int64_t)ev[e] * W;
         int32_t k = 0;
-        for (int64_t w = 0; w < W; w++) k += __builtin_popcountll(ra[w].bits & rb[w].bits);
+        each_common(e, [&](int64_t, int32_t, int32_t) { k++; });
         g.tcnt[e] = k;
       });
       for (int64_t e = 0; e < ne; e++) cap[e + 1] = cap[e] + g.tcnt[e];
@@ -371,26 +402,17 @@ void collapse_edges(int64_t ne, const int32_t* u, const int32_t* v, uint8_t* kep
     }
     if (cap[ne] <= kTriListMax) {
       // kept by the calling thread between calls: fresh pages cost more than filling them
-      thread_local TriBuffer keep;
+      thread_local Pages<Tri> keep;
       keep.reserve((size_t)cap[ne]);
       g.tri = keep.p;
       if (!g.simple) g.tx.resize((size_t)cap[ne]);
       if (nv <= kBitsetVertices) {
         parallel_edges([&](int64_t e) {
-          const int32_t a = eu[e], b = ev[e];
-          const Graph::Word *ra = nb.data() + (int64_t)a * W, *rb = nb.data() + (int64_t)b * W;
           Tri* tri = g.tri + cap[e];
-          for (int64_t w = 0; w < W; w++) {
-            uint64_t m = ra[w].bits & rb[w].bits;
-            while (m) {
-              const int bit = __builtin_ctzll(m);
-              const uint64_t below = (1ull << bit) - 1;
-              if (!g.simple) g.tx[(size_t)(tri - g.tri)] = (int32_t)(w * 64 + bit);
-              *tri++ = Tri{g.eid[ra[w].pos + __builtin_popcountll(ra[w].bits & below)],
-                           g.eid[rb[w].pos + __builtin_popcountll(rb[w].bits & below)]};
-              m &= m - 1;
-            }
-          }
+          each_common(e, [&](int64_t x, int32_t ea, int32_t eb) {
+            if (!g.simple) g.tx[(size_t)(tri - g.tri)] = (int32_t)x;
+            *tri++ = Tri{ea, eb};
+          });
         });
       } else {
         parallel_edges([&](int64_t e) {
