@@ -36,6 +36,20 @@
 
 #include "ssq_internal.h"
 
+// This file is built twice.  The tests count bits throughout, so the second build, with
+// SSQ_COLLAPSE_POPCNT defined, may use the processor's instruction for it; the first one has the entry
+// points and calls the second's collapse where it is linked in and the processor has that instruction
+// (4096 rotations at mean degree 80: 47 ms in all with it, 57.5 without).
+namespace ssq {
+#ifdef SSQ_COLLAPSE_POPCNT
+#define SSQ_COLLAPSE collapse_edges_popcnt
+#else
+#define SSQ_COLLAPSE collapse_edges_plain
+static
+#endif
+void SSQ_COLLAPSE(int64_t ne, const int32_t* u, const int32_t* v, uint8_t* kept, int threads);
+}
+
 namespace {
 
 // Uninitialised storage in large pages where the system has them, grown as needed and never shrunk.
@@ -258,7 +272,7 @@ bool dominated(const Graph& g, int32_t e, Valid valid, Work& wk, int32_t* witnes
 
 namespace ssq {
 
-void collapse_edges(int64_t ne, const int32_t* u, const int32_t* v, uint8_t* kept, int threads) {
+void SSQ_COLLAPSE(int64_t ne, const int32_t* u, const int32_t* v, uint8_t* kept, int threads) {
   if (ne <= 0) return;
   // compact vertex labels to 0..nv-1 in increasing label order
   int32_t lmin = u[0], lmax = u[0];
@@ -541,9 +555,20 @@ void collapse_edges(int64_t ne, const int32_t* u, const int32_t* v, uint8_t* kep
 
 }  // namespace ssq
 
+#ifndef SSQ_COLLAPSE_POPCNT
+namespace ssq {
+__attribute__((weak)) void collapse_edges_popcnt(int64_t ne, const int32_t* u, const int32_t* v, uint8_t* kept,
+                                                 int threads);
+}
+void ssq::collapse_edges(int64_t ne, const int32_t* u, const int32_t* v, uint8_t* kept, int threads) {
+  if (collapse_edges_popcnt && __builtin_cpu_supports("popcnt")) collapse_edges_popcnt(ne, u, v, kept, threads);
+  else collapse_edges_plain(ne, u, v, kept, threads);
+}
+
 extern "C" int ssq_collapse_edges(int64_t ne, const int32_t* u, const int32_t* v, uint8_t* kept, int threads) {
   if (ne < 0 || (ne > 0 && (!u || !v || !kept))) return SSQ_EINVAL;
   if (threads <= 0) threads = (int)std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
   ssq::collapse_edges(ne, u, v, kept, threads);
   return SSQ_OK;
 }
+#endif
