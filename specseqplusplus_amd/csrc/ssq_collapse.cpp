@@ -52,7 +52,7 @@ void SSQ_COLLAPSE(int64_t ne, const int32_t* u, const int32_t* v, uint8_t* kept,
 
 namespace {
 
-// Uninitialised storage in large pages where the system has them, grown as needed and never shrunk.
+// Uninitialised storage in large pages where the system has them, grown as needed.
 template <typename T>
 struct Pages {
   T* p = nullptr;
@@ -60,13 +60,17 @@ struct Pages {
   Pages() = default;
   Pages(const Pages&) = delete;
   Pages& operator=(const Pages&) = delete;
-  ~Pages() { std::free(p); }
+  ~Pages() { release(); }
+  void release() {
+    std::free(p);
+    p = nullptr;
+    cap = 0;
+  }
   void reserve(size_t n) {
     if (n <= cap) return;
     constexpr size_t kPage = size_t(1) << 21;
     const size_t bytes = ((n + n / 4) * sizeof(T) + kPage - 1) / kPage * kPage;
-    std::free(p);
-    cap = 0;
+    release();
     p = (T*)std::aligned_alloc(kPage, bytes);
     if (!p) throw std::bad_alloc();
     madvise(p, bytes, MADV_HUGEPAGE);  // a hint: without it only slower
@@ -88,6 +92,7 @@ struct Graph {
   // 9 of 44 triangles are valid in the tests of 4096 rotations at mean degree 80), so they hold
   // both ids side by side and not x, which is read off (a, x) for the valid ones.
   std::vector<int64_t> toff;
+  Pages<Tri> own;      // the lists, where they are not kept between calls
   Tri* tri = nullptr;  // edge e's triangles: [toff[e], toff[e] + tcnt[e])
   std::vector<int32_t> tcnt;
   // No loops and no two edges with the same ends.  Otherwise the tables have more than one answer
@@ -108,6 +113,7 @@ struct Graph {
   int64_t W = 0;
 };
 constexpr int64_t kTriListMax = int64_t(1) << 28;  // entries (8 bytes each)
+constexpr size_t kTriKeep = size_t(1) << 25;       // of them kept by a thread between calls (256 MB)
 constexpr int64_t kBitsetVertices = 16384;          // neighbourhood bit sets up to 64 MB
 
 template <typename Valid>
@@ -415,10 +421,12 @@ void SSQ_COLLAPSE(int64_t ne, const int32_t* u, const int32_t* v, uint8_t* kept,
         cap[e + 1] = cap[e] + std::min(g.off[eu[e] + 1] - g.off[eu[e]], g.off[ev[e] + 1] - g.off[ev[e]]);
     }
     if (cap[ne] <= kTriListMax) {
-      // kept by the calling thread between calls: fresh pages cost more than filling them
+      // Kept by the calling thread between calls, as fresh pages cost more than filling them; above
+      // kTriKeep the search takes so much longer that the pages are given back at the end of the call.
       thread_local Pages<Tri> keep;
-      keep.reserve((size_t)cap[ne]);
-      g.tri = keep.p;
+      Pages<Tri>& lists = (size_t)cap[ne] <= kTriKeep ? keep : g.own;
+      lists.reserve((size_t)cap[ne]);
+      g.tri = lists.p;
       if (!g.simple) g.tx.resize((size_t)cap[ne]);
       if (nv <= kBitsetVertices) {
         parallel_edges([&](int64_t e) {
