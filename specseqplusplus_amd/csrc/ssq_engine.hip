@@ -1123,20 +1123,46 @@ __device__ __forceinline__ uint32_t next_step(const Dev& d, const uint32_t* bits
   }
 }
 
-// f(row - lo) for every row of a pivot, spread over kThreads threads with kU loads in flight each.
-template <int kThreads, int kU, typename F>
-__device__ __forceinline__ void toggle_rows(const int32_t* B, int32_t len, int t, int32_t lo, F f) {
-  for (int32_t k0 = t; k0 < len; k0 += kThreads * kU) {
+// f(row - lo) for every row of a pivot, spread over some threads (t: this one's place among them) with
+// kU loads in flight each.
+template <int kU, typename F>
+__device__ __forceinline__ void toggle_rows(const int32_t* B, int32_t len, int t, int threads, int32_t lo, F f) {
+  for (int32_t k0 = t; k0 < len; k0 += threads * kU) {
     int32_t x[kU];
 #pragma unroll
     for (int u = 0; u < kU; u++) {
-      const int32_t k = k0 + u * kThreads;
+      const int32_t k = k0 + u * threads;
       x[u] = k < len ? B[k] - lo : -1;
     }
 #pragma unroll
     for (int u = 0; u < kU; u++)
       if (x[u] >= 0) f(x[u]);
   }
+}
+
+// The pivots of a step, a wavefront each; where there are fewer than wavefronts, two, four or all of them
+// share one (2000 apparent pivots of 1000 rows, one to a step, in k_add_long: 10.2 ms with a wavefront each,
+// 4.3 ms so; one addition at a time took 4.5 ms).  Returns this thread's part of the bytes read.
+template <typename F>
+__device__ __forceinline__ unsigned long long toggle_picks(const Dev& d, const Picks& P, uint32_t n, int32_t lo, F f) {
+  constexpr int kWaves = kLongThreads / kWave;
+  const int wave = uniform(threadIdx.x / kWave);
+  unsigned long long bytes = 0;
+  if (n > kWaves / 2) {
+    for (uint32_t e = wave; e < n; e += kWaves) {
+      const int32_t len = uniform(P.list[e].len);
+      toggle_rows<8>(d.pool + uniform64(P.list[e].off), len, lane_id(), kWave, lo, f);
+      bytes += 4ull * (unsigned long long)len + 24ull;  // the pivot read; the bit set stays on chip
+    }
+  } else {
+    const int sh = n > 2 ? 1 : n == 2 ? 2 : 3, e = wave >> sh, part = wave & ((1 << sh) - 1);
+    if (e < (int)n) {
+      const int32_t len = uniform(P.list[e].len);
+      toggle_rows<8>(d.pool + uniform64(P.list[e].off), len, part * kWave + lane_id(), kWave << sh, lo, f);
+      if (part == 0) bytes = 4ull * (unsigned long long)len + 24ull;
+    }
+  }
+  return bytes;
 }
 
 // Every set bit of the words [w0, w1) of a source, in order: each wavefront takes a contiguous part,
@@ -1257,13 +1283,7 @@ __global__ void __launch_bounds__(kLongThreads) k_add_long(Dev d, int r, int32_t
         if (t & 1u) {
           n = min(n, (uint32_t)kPicks);
           reach = next_reach(reach, n, chain);
-          for (uint32_t e = tid / kWave; e < n; e += kLongThreads / kWave) {
-            const int32_t len = picks.list[e].len;
-            toggle_rows<kWave, 8>(d.pool + picks.list[e].off, len, lane_id(), lo, [&](int32_t x) {
-              atomicXor(&bits[x >> 5], 1u << (x & 31));
-            });
-            n_bytes += 4ull * (unsigned long long)len + 24ull;  // the pivot read; the bit set is in LDS
-          }
+          n_bytes += toggle_picks(d, picks, n, lo, [&](int32_t x) { atomicXor(&bits[x >> 5], 1u << (x & 31)); });
           chain += n;
         } else {
           const uint32_t p = (uint32_t)__builtin_amdgcn_readfirstlane((int)d.piv[l]);
@@ -1274,7 +1294,7 @@ __global__ void __launch_bounds__(kLongThreads) k_add_long(Dev d, int r, int32_t
             to_huge = true;
             break;
           }
-          toggle_rows<kLongThreads, 16>(d.pool + pm.off, pm.len, tid, lo, [&](int32_t x) {
+          toggle_rows<16>(d.pool + pm.off, uniform(pm.len), tid, kLongThreads, lo, [&](int32_t x) {
             atomicXor(&bits[x >> 5], 1u << (x & 31));
           });
           if (tid < kWave) n_bytes += 4ull * (unsigned long long)pm.len + 24ull;
@@ -1582,11 +1602,7 @@ __global__ void __launch_bounds__(kLongThreads) k_add_huge(Dev d, int r, int32_t
         if (t & 1u) {  // the low's pivot and those of the rows near it
           n = min(n, (uint32_t)kPicks);
           reach = next_reach(reach, n, chain);
-          for (uint32_t e = tid / kWave; e < n; e += kLongThreads / kWave) {
-            const int32_t len = picks.list[e].len;
-            toggle_rows<kWave, 8>(d.pool + picks.list[e].off, len, lane_id(), lo, toggle);
-            n_bytes += 4ull * (unsigned long long)len + 24ull;  // the pivot read; the bit set stays on chip
-          }
+          n_bytes += toggle_picks(d, picks, n, lo, toggle);
           chain += n;
           n_add += n;
           __syncthreads();
@@ -1613,7 +1629,7 @@ __global__ void __launch_bounds__(kLongThreads) k_add_huge(Dev d, int r, int32_t
         dense = false;
       }
       if (dense) {
-        toggle_rows<kLongThreads, 16>(B, b_len, tid, lo, toggle);
+        toggle_rows<16>(B, b_len, tid, kLongThreads, lo, toggle);
         if (tid == 0) atomicMin(&picks.minw, (b_first - lo) >> 5);
         n_add += 1;
         if (tid < kWave) n_bytes += 4ull * (unsigned long long)b_len + 24ull;
