@@ -120,26 +120,33 @@ template <typename Valid>
 int64_t common(const Graph& g, int32_t a, int32_t b, Valid valid, int32_t* out, int32_t* ea,
                int32_t* eb);
 
-// Valid common neighbours of edge e (ascending), with the two edge ids.
+// ... without triangle lists, or of a list that is not simple (out of line: the ordinary test is short).
 template <typename Valid>
-int64_t common_e(const Graph& g, int32_t e, Valid valid, int32_t* out, int32_t* ea, int32_t* eb) {
-  if (g.toff.empty()) return common(g, g.eu[e], g.ev[e], valid, out, ea, eb);
+__attribute__((noinline)) int64_t common_any(const Graph& g, int32_t e, Valid valid, int32_t* out, int32_t* ea,
+                                             int32_t* eb, bool ids) {
+  if (g.toff.empty()) return common(g, g.eu[e], g.ev[e], valid, out, ids ? ea : nullptr, ids ? eb : nullptr);
+  int64_t k = 0;
+  const int32_t* tx = g.tx.data() + g.toff[e];
+  const Tri* tri = g.tri + g.toff[e];
+  for (int32_t t = 0, nt = g.tcnt[e]; t < nt; t++) {
+    const int32_t e1 = tri[t].ea, e2 = tri[t].eb;
+    if (!valid(e1) || !valid(e2)) continue;
+    ea[k] = e1;
+    eb[k] = e2;
+    out[k++] = tx[t];
+  }
+  return k;
+}
+
+// Valid common neighbours of edge e (ascending), with the two edge ids (not in every case without ids).
+template <typename Valid>
+int64_t common_e(const Graph& g, int32_t e, Valid valid, int32_t* out, int32_t* ea, int32_t* eb, bool ids) {
+  if (__builtin_expect(g.toff.empty() | !g.simple, 0)) return common_any(g, e, valid, out, ea, eb, ids);
   int64_t k = 0;
   const Tri* tri = g.tri + g.toff[e];
   const int32_t nt = g.tcnt[e], a = g.eu[e];
   // No branch on what is valid, which cannot be predicted: every entry is written, and k stands
   // still for those that are not (an edge has fewer triangles than the arrays have room).
-  if (!g.simple) {
-    const int32_t* tx = g.tx.data() + g.toff[e];
-    for (int32_t t = 0; t < nt; t++) {
-      const int32_t e1 = tri[t].ea, e2 = tri[t].eb;
-      if (!valid(e1) || !valid(e2)) continue;
-      ea[k] = e1;
-      eb[k] = e2;
-      out[k++] = tx[t];
-    }
-    return k;
-  }
   for (int32_t t = 0; t < nt; t++) {
     const int32_t e1 = tri[t].ea, e2 = tri[t].eb;
     ea[k] = e1;
@@ -161,8 +168,10 @@ int64_t common(const Graph& g, int32_t a, int32_t b, Valid valid, int32_t* out, 
     if (x < y) i++;
     else if (x > y) j++;
     else {
-      ea[k] = g.eid[i];
-      eb[k] = g.eid[j];
+      if (ea) {
+        ea[k] = g.eid[i];
+        eb[k] = g.eid[j];
+      }
       if (out) out[k] = x;
       k++;
       i++;
@@ -217,12 +226,25 @@ inline int32_t uncovered(const Graph& g, int32_t w, const int32_t* I, int64_t m,
 struct Work {
   std::vector<int32_t> I, C, ea, eb;
   int64_t m = 0;
-  explicit Work(int64_t maxdeg) : I((size_t)maxdeg), C((size_t)maxdeg), ea((size_t)maxdeg), eb((size_t)maxdeg) {}
+  bool ids;  // the edges are read afterwards
+  Work(int64_t maxdeg, bool ids_read) : I((size_t)maxdeg), C((size_t)maxdeg), ea((size_t)maxdeg), eb((size_t)maxdeg), ids(ids_read) {}
 };
+template <typename Valid>
+__attribute__((noinline)) bool dominated_in_turn(const Graph& g, const int32_t* I, int64_t m, Valid valid,
+                                                 int32_t* witness) {
+  const int32_t hint = *witness;
+  if (hint >= 0 && std::binary_search(I, I + m, hint) && uncovered(g, hint, I, m, valid) < 0) return true;
+  for (int64_t c = 0; c < m; c++) {
+    if (I[c] == hint || uncovered(g, I[c], I, m, valid) >= 0) continue;
+    *witness = I[c];
+    return true;
+  }
+  return false;
+}
 template <typename Valid>
 bool dominated(const Graph& g, int32_t e, Valid valid, Work& wk, int32_t* witness, int32_t missed) {
   int32_t *I = wk.I.data(), *C = wk.C.data();
-  const int64_t m = wk.m = common_e(g, e, valid, I, wk.ea.data(), wk.eb.data());
+  const int64_t m = wk.m = common_e(g, e, valid, I, wk.ea.data(), wk.eb.data(), wk.ids);
   if (m <= 1) {
     if (m == 1) *witness = I[0];
     return m == 1;
@@ -230,16 +252,7 @@ bool dominated(const Graph& g, int32_t e, Valid valid, Work& wk, int32_t* witnes
   // Striking relies on an edge having one id from both its ends, and on the bit sets: without them an id
   // is a binary search, and it pays to read one candidate's list after the other (17,000 vertices of
   // mean degree 300: 5.6 s with the searches, 5.2 s this way, on 8 threads; in the plane 2.3 and 1.7 s).
-  if (!g.simple || !g.W) {
-    const int32_t hint = *witness;
-    if (hint >= 0 && std::binary_search(I, I + m, hint) && uncovered(g, hint, I, m, valid) < 0) return true;
-    for (int64_t c = 0; c < m; c++) {
-      if (I[c] == hint || uncovered(g, I[c], I, m, valid) >= 0) continue;
-      *witness = I[c];
-      return true;
-    }
-    return false;
-  }
+  if (__builtin_expect(!g.simple | !g.W, 0)) return dominated_in_turn(g, I, m, valid, witness);
   int64_t n = m;
   std::copy(I, I + m, C);
   auto strike = [&](int32_t x) {  // x stays a candidate, and those joined to it by a valid edge
@@ -458,7 +471,7 @@ void SSQ_COLLAPSE(int64_t ne, const int32_t* u, const int32_t* v, uint8_t* kept,
   {
     std::atomic<int64_t> next{1};
     auto work = [&]() {
-      Work wk(maxdeg);
+      Work wk(maxdeg, false);
       for (;;) {
         int64_t s = next.fetch_add(256);
         if (s >= ne) break;
@@ -477,7 +490,7 @@ void SSQ_COLLAPSE(int64_t ne, const int32_t* u, const int32_t* v, uint8_t* kept,
 
   // 2. sequential cascades
   g.crit.assign((size_t)ne, 0);
-  Work wk(maxdeg);
+  Work wk(maxdeg, true);
   std::priority_queue<int32_t> heap;
   // vertices that may have become common neighbours of a pushed edge since its last test: a
   // list per edge in a pool that lives for one cascade (every pushed edge is popped in it)
@@ -503,7 +516,7 @@ void SSQ_COLLAPSE(int64_t ne, const int32_t* u, const int32_t* v, uint8_t* kept,
     const uint8_t* crit = g.crit.data();
     if (!g.simple)  // an edge may be in a triangle of its own: the test before did not see it as critical
       wk.m = common_e(g, e, [thresh, crit](int32_t x) { return (x < thresh) | crit[x]; }, wk.I.data(), wk.ea.data(),
-                      wk.eb.data());
+                      wk.eb.data(), true);
     const int32_t p = g.eu[e], q = g.ev[e];
     for (int64_t k = 0; k < wk.m; k++) {
       const int32_t e1 = wk.ea[k], e2 = wk.eb[k];  // e1 = (p, x) gains q, e2 = (q, x) gains p
@@ -539,7 +552,7 @@ void SSQ_COLLAPSE(int64_t ne, const int32_t* u, const int32_t* v, uint8_t* kept,
     g.crit[idx] = 1;
     kept[idx] = 1;
     wk.m = common_e(g, idx, [idx, crit = g.crit.data()](int32_t x) { return (x < idx) | crit[x]; }, wk.I.data(),
-                    wk.ea.data(), wk.eb.data());
+                    wk.ea.data(), wk.eb.data(), true);
     three_clique(idx, idx, idx);
     while (!heap.empty()) {
       int32_t cur = heap.top();
