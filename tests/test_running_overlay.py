@@ -123,7 +123,7 @@ def returning(base_len, b_len, spread, seed):
     return column, pivots
 
 
-def review_column():
+def ranges_column():
     """The cleared rows 69-40 under lows 1000-994, then 69 back: 69 overlay lanes."""
     r = lambda a, b: set(range(a, b + 1))
     pivots = [{1000, 999, 998, 997} | r(500, 511), {999} | r(55, 69), {998} | r(40, 54),
@@ -139,7 +139,7 @@ def steps_column():
     return set(R), pivots
 
 
-CASES = {"review": review_column(), "steps": steps_column(), "steps_on": (steps_column()[0], steps_column()[1] + [{599, 200}])}
+CASES = {"ranges": ranges_column(), "steps": steps_column(), "steps_on": (steps_column()[0], steps_column()[1] + [{599, 200}])}
 for _len in (63, 64, 65, 66, 128, 129, 200):
     for _b in (2, 3, 5, 6, 7, 8, 15, 16):
         CASES[f"len{_len}_rows{_b}"] = returning(_len, _b, (_len + _b) % 3 if _b > 5 else _b // 5, _len * 100 + _b)
@@ -170,7 +170,7 @@ def test_rows_below_the_top_alone_are_not_enough():
             chase(column, pivots, below_low=False)
         except Overflow:
             over.append(name)
-    assert {"review", "steps", "steps_on"} <= set(over) and len(over) > 10
+    assert {"ranges", "steps", "steps_on"} <= set(over) and len(over) > 10
 
 
 def test_guard_holds_on_random_pivots():
@@ -205,7 +205,7 @@ def test_returning_rows(h, name):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("name", ["review", "steps", "len63_rows16", "len64_rows2", "len200_rows15"])
+@pytest.mark.parametrize("name", ["ranges", "steps", "len63_rows16", "len64_rows2", "len200_rows15"])
 def test_bytes_of_a_chase(h, name):
     """add_bytes is 4(|a| + |b| + |a ^ b|) + 24 for each addition of the one chase (no row of these
     columns is in the overlay and in the base at once)."""
